@@ -61,6 +61,30 @@ def test_vector_codec_bit_exact(D, O, G):
     assert np.array_equal(host_bits(back).ravel(), orc.kivi_decompress(want, n, D, O, G))
 
 
+@pytest.mark.parametrize("D,O,G", [(128, 63, 2), (128, 0, 2), (127, 9, 14), (128, 17, 30), (65, 33, 4),
+                                   (8, 8, 4), (3, 1, 1000)])
+@pytest.mark.parametrize("n,skew", [(1, 0), (8, 0), (21, 1)])
+def test_vector_codec_slot_counts_and_alignment(D, O, G, n, skew):
+    """Outlier counts either side of a lane's slots, the longest record, last
+    groups of one channel, partial workgroups, and bases off the wide
+    accesses' alignment; the bytes past a record stay."""
+    rng = np.random.default_rng(D * 7 + O + n)
+    xb = np.ascontiguousarray(_f16(_special_vectors(rng, max(n, 16), (D + 9) // 2 * 2))[:n, :D])
+    stride = orc.kivi_compressed_bytes(D, O, G)
+    want = np.full(n * stride, 0xAB, np.uint8)
+    orc.kivi_compress(xb, D, O, G, out=want)
+    print(f"case vec codec D={D} O={O} G={G} n={n} skew={skew}", flush=True)
+    x = torch.zeros(n * D + skew, dtype=torch.float16, device="cuda")[skew:]
+    x.copy_(dev(xb, orc.F16).view(-1))
+    rec = torch.full((n * stride + skew,), 0xAB, dtype=torch.uint8, device="cuda")[skew:]
+    tla.kivi_compress(x, rec, n, D, O, G)
+    back = torch.zeros(n * D + skew, dtype=torch.float16, device="cuda")[skew:]
+    tla.kivi_decompress(rec, back, n, D, O, G)
+    torch.cuda.synchronize()
+    assert np.array_equal(rec.cpu().numpy(), want)
+    assert np.array_equal(host_bits(back).ravel(), orc.kivi_decompress(want, n, D, O, G).ravel())
+
+
 def test_vector_codec_hand_derived_slot_order():
     """The kernel writes the outliers in the reference's selection-slot order
     (kivi_cache.cu:50-78), byte for byte against records derived by hand
