@@ -7,6 +7,7 @@ import inputs
 import oracle_lib as orc
 import tl_attn as tla
 from gpu_util import dev, host_bits
+from test_oracle import rope_tables
 
 pytestmark = pytest.mark.gpu
 
@@ -177,3 +178,73 @@ def test_convert_fp8_other_sources_and_unaligned_tails(code):
         nan = (w & 0x7F) == 0x7F
         assert np.array_equal(g[~nan], w[~nan]) and ((g[nan] & 0x7F) == 0x7F).all()
         assert (got[:off] == 0xAB).all() and (got[off + n:] == 0xAB).all()
+
+
+def _prompt_slots(rng, BS, spans):
+    """Slots of prompts of (first position, tokens), each over blocks of its own in any order; then breaks:
+    padded tokens, a token past the pool, a run written backwards, a jump inside a block."""
+    blocks = sum((a + n + BS - 1) // BS for a, n in spans)
+    N = blocks + 3
+    order, at, out = rng.permutation(N), 0, []
+    for a, n in spans:
+        pos = np.arange(a, a + n)
+        out.append(order[at + pos // BS] * BS + pos % BS)
+        at += (a + n + BS - 1) // BS
+    s = np.concatenate(out).astype(np.int32)
+    s[70:73] = -1
+    s[101] = N * BS + 3
+    s[128:140] = s[128:140][::-1].copy()
+    s[150], s[158] = s[158], s[150]
+    return s, N
+
+
+@pytest.mark.parametrize("kind", ["copy", "halves", "adjacent", "fp8"])
+@pytest.mark.parametrize("code", [orc.F16, orc.BF16, orc.F32])
+@pytest.mark.parametrize("n_kv,D,BS", [(2, 128, 16), (3, 64, 8), (1, 128, 24), (2, 112, 40), (1, 256, 64), (2, 128, 12)])
+def test_prompt_append_bit_exact(kind, code, n_kv, D, BS):
+    """More than 256 tokens: whole 16-byte chunks of a block's rows where tokens fill them, elements elsewhere.
+    Prompts begin anywhere in a block and end a tile early, on it and past it; 12-slot blocks take the
+    general kernel."""
+    if kind == "fp8" and code == orc.F32:
+        pytest.skip("FP8 pools take 2-byte sources")
+    rng = np.random.default_rng(D * BS + n_kv)
+    spans = [(5, 163), (0, 33), (BS - 1, 64), (3, 1), (0, BS), (17, 95)]
+    slots, N = _prompt_slots(rng, BS, spans)
+    T, H = slots.size, 5
+    key = inputs.encode(rng.standard_normal((T, n_kv, D), dtype=np.float32), code)
+    val = inputs.encode(rng.standard_normal((T, n_kv, D), dtype=np.float32), code)
+    ok = np.where(slots < N * BS, slots, -1).astype(np.int32)
+    print(f"case prompt append {kind} code={code} T={T} n_kv={n_kv} D={D} BS={BS}", flush=True)
+    if kind == "fp8":
+        k8 = rng.integers(0, 255, (N, n_kv, D, BS), dtype=np.uint8)
+        v8 = k8[::-1].copy()
+        kd8, vd8 = torch.from_numpy(k8.copy()).cuda(), torch.from_numpy(v8.copy()).cuda()
+        tla.reshape_and_cache_fp8(dev(key, code), dev(val, code), kd8, vd8, dev(slots), 3.1 / 448, 0.02)
+        torch.cuda.synchronize()
+        orc.reshape_and_cache_fp8(key, val, code, k8, v8, ok, 3.1 / 448, 0.02)
+        assert np.array_equal(kd8.cpu().numpy(), k8)
+        assert np.array_equal(vd8.cpu().numpy(), v8)
+        return
+    kc = inputs.encode(rng.standard_normal((N, n_kv, D, BS), dtype=np.float32), code)
+    vc = inputs.encode(rng.standard_normal((N, n_kv, D, BS), dtype=np.float32), code)
+    kcd, vcd = dev(kc, code), dev(vc, code)
+    if kind == "copy":
+        tla.reshape_and_cache_split(dev(key, code), dev(val, code), kcd, vcd, dev(slots))
+        torch.cuda.synchronize()
+        orc.reshape_and_cache(key, val, kc, vc, ok)
+    else:
+        style = tla.ROPE_HALVES if kind == "halves" else tla.ROPE_ADJACENT
+        q = inputs.encode(rng.standard_normal((T, H, D), dtype=np.float32), code)
+        pos = rng.integers(0, 500, T).astype(np.int32)
+        pos[45], pos[200] = 500, -1                      # past the tables: nothing written
+        cos_t, sin_t = rope_tables(500, D)
+        qd = dev(q, code)
+        q_out = torch.zeros_like(qd)
+        tla.rope_reshape_and_cache(qd, dev(key, code), dev(val, code), kcd, vcd, dev(slots), dev(pos), dev(cos_t),
+                                   dev(sin_t), style, q_out=q_out)
+        torch.cuda.synchronize()
+        q_ref = np.zeros_like(q)
+        orc.rope_reshape_and_cache(q, q_ref, key, val, kc, vc, ok, pos, cos_t, sin_t, code, style)
+        assert np.array_equal(host_bits(q_out), q_ref)
+    assert np.array_equal(host_bits(kcd), kc)
+    assert np.array_equal(host_bits(vcd), vc)

@@ -158,7 +158,9 @@ __global__ __launch_bounds__(64) void reshape_rows_kernel(
 }
 
 // The row kernel serves calls of at most this many tokens (each wavefront
-// scans the call's slots for a shared block).
+// scans the call's slots for a shared block).  One token per block, copied:
+// 256 tokens 7.0 us here, 8.5 in append_tiles_kernel; 64 tokens 3.6 and 6.4.
+// From 256 prompt tokens on the tiles win: 300 tokens 4.1 against 7.0 us.
 constexpr int kRowAppendMaxTokens = 256;
 
 template <Kind SRC>
@@ -403,6 +405,264 @@ __global__ __launch_bounds__(64) void rope_rows_kernel(RopeCache a) {
   }
 }
 
+// Prompt-sized appends.  The element stores of reshape_copy_kernel and
+// rope_cache_kernel leave one 2-byte store per (token, channel), each
+// instruction over 64 lines of the pool.  Here a workgroup takes a tile of 32
+// consecutive tokens of one kv head, of K or of V, stages their rows in LDS
+// and writes the pool along the slots: where C = 16 / E tokens of the tile
+// fill an aligned 16-byte chunk, it is one store per channel, with the lanes
+// of a store over consecutive chunks of a block's rows; tokens that fill no
+// chunk are stored element by element, and no slot of another token is
+// written.
+//
+// Tokens belong to segments: consecutive tokens of the call in consecutive
+// slots of one aligned group of `group` slots (at most 32: a block or a part
+// of one).  A tile takes the segments that begin in it, so that a group's
+// lines have one writer, and at most 32 + 31 tokens, whose slots fit a
+// wavefront's lanes.
+//
+// Bound by HBM.  4180 tokens of 8 kv heads, 32 heads, d 128, bf16, blocks of
+// 16, rotated: 28.2 us (element stores: 93.7); 4096 tokens copied without
+// rotation 7.9 us (43.2), into FP8 pools 8.3 us (42.8).  Tokens that each lie
+// in a block of their own (a decode batch of more than 256 sequences) are
+// stored element by element as before: 512 of them copied 10.4 us (9.8),
+// 1024 17.1 (17.5).
+struct TileAppend {
+  const void* q; void* q_out;              // ROPE only
+  const void* key; const void* value;
+  char* k_cache; char* v_cache;
+  const int32_t* slots; const int32_t* positions;
+  const float* cos_table; const float* sin_table;
+  int num_tokens, num_heads, num_kv_heads, head_size, block_size, num_blocks, max_positions;
+  int group;                               // slots of a segment's group
+  int kv_wgs;                              // workgroups over K and V; q's follow
+  float k_mul, v_mul;                      // FP8 pools
+};
+
+constexpr int kTileTokens = 32, kTileThreads = 256, kTileRowPad = 8;
+constexpr int kTileHeadsPerThread = 4;     // q heads of one token and rotation unit
+constexpr int kNoRope = -1;
+
+// Eight elements of a row in the pool's type, staged in LDS (8-byte aligned).
+template <Kind POOL>
+__device__ __forceinline__ void stage8(char* dst, const float* x) {
+  uint32_t* d = reinterpret_cast<uint32_t*>(dst);
+  if constexpr (POOL == Kind::FP8) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) d[i] = pack4_fp8(x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]);
+  } else if constexpr (POOL == Kind::F32) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) d[i] = scalar_bits<POOL>(x[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = scalar_bits<POOL>(x[2 * i]) | scalar_bits<POOL>(x[2 * i + 1]) << 16;
+  }
+}
+
+// Eight elements in fp32.
+template <Kind K>
+__device__ __forceinline__ void load8f(const void* p, int64_t i, float* f) {
+  if constexpr (K == Kind::F32) {
+    const u32x4 a = load16((const float*)p + i), b = load16((const float*)p + i + 4);
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = __uint_as_float(w[e]);
+  } else {
+    load8<K>(p, i, f);
+  }
+}
+
+// Rotation unit u of a row at `base`: pairs 8 u .. 8 u + 7, their elements
+// in lo (ADJACENT: the first 8 of 16 consecutive ones; HALVES: the first of
+// each pair) and hi.
+template <Kind K, int STYLE>
+__device__ __forceinline__ void load_unit(const void* p, int64_t base, int u, int half, float* lo, float* hi) {
+  load8f<K>(p, base + (STYLE == 0 ? 16 * u : 8 * u), lo);
+  load8f<K>(p, base + (STYLE == 0 ? 16 * u + 8 : half + 8 * u), hi);
+}
+template <int STYLE>
+__device__ __forceinline__ void rotate_unit(float* lo, float* hi, const float* c, const float* s) {
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {
+    float& a = STYLE == 0 ? (p < 4 ? lo[2 * p] : hi[2 * p - 8]) : lo[p];
+    float& b = STYLE == 0 ? (p < 4 ? lo[2 * p + 1] : hi[2 * p - 7]) : hi[p];
+    const float x0 = a, x1 = b;
+    a = fp32_result(__builtin_fmaf(x0, c[p], -(x1 * s[p])));
+    b = fp32_result(__builtin_fmaf(x0, s[p], x1 * c[p]));
+  }
+}
+
+template <Kind K, int STYLE>
+__device__ __forceinline__ void rotate_q_tile(const TileAppend& a, int wg) {
+  const int half = a.head_size / 2, units = half / 8;
+  const int sets = (a.num_heads + kTileHeadsPerThread - 1) / kTileHeadsPerThread;
+  const int64_t idx = (int64_t)wg * kTileThreads + threadIdx.x;
+  const int u = (int)(idx % units);
+  const int set = (int)((idx / units) % sets);
+  const int64_t t = idx / ((int64_t)units * sets);
+  if (t >= a.num_tokens) return;
+  const int pos = a.positions[t];
+  if (pos < 0 || pos >= a.max_positions) return;                // token left as it is
+  float c[8], s[8], lo[kTileHeadsPerThread][8], hi[kTileHeadsPerThread][8];
+  load8f<Kind::F32>(a.cos_table, (int64_t)pos * half + 8 * u, c);
+  load8f<Kind::F32>(a.sin_table, (int64_t)pos * half + 8 * u, s);
+  // head set + sets i: the lanes of a wavefront on consecutive heads
+#pragma unroll
+  for (int i = 0; i < kTileHeadsPerThread; ++i) {
+    const int h = set + i * sets;
+    if (h < a.num_heads)
+      load_unit<K, STYLE>(a.q, (t * a.num_heads + h) * a.head_size, u, half, lo[i], hi[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < kTileHeadsPerThread; ++i) {
+    const int h = set + i * sets;
+    if (h >= a.num_heads) break;
+    rotate_unit<STYLE>(lo[i], hi[i], c, s);
+    const int64_t base = (t * a.num_heads + h) * a.head_size;
+    constexpr int E = KindInfo<K>::bytes;
+    alignas(16) char row[8 * E];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      stage8<K>(row, j ? hi[i] : lo[i]);
+      const int64_t at = base + (STYLE == 0 ? 16 * u + 8 * j : j * half + 8 * u);
+#pragma unroll
+      for (int w = 0; w < E / 2; ++w)
+        *reinterpret_cast<u32x4*>((char*)a.q_out + at * E + 16 * w) = reinterpret_cast<const u32x4*>(row)[w];
+    }
+  }
+}
+
+template <Kind SRC, Kind POOL, int ROPE>
+__global__ __launch_bounds__(kTileThreads) void append_tiles_kernel(TileAppend a) {
+  extern __shared__ char tile_rows[];
+  if constexpr (ROPE != kNoRope) {
+    if ((int)blockIdx.x >= a.kv_wgs) {
+      rotate_q_tile<SRC, ROPE>(a, blockIdx.x - a.kv_wgs);
+      return;
+    }
+  }
+  constexpr int E = KindInfo<POOL>::bytes, C = 16 / E;
+  const int h = (int)(blockIdx.x / 2) % a.num_kv_heads, t0 = (int)(blockIdx.x / 2) / a.num_kv_heads * kTileTokens;
+  const bool is_v = blockIdx.x % 2;
+  const int tid = threadIdx.x, lane = tid % kWave;
+
+  // lane i: token t0 + i, and the token before it
+  auto slot_of = [&](int t) {
+    if (t < 0 || t >= a.num_tokens) return -1;
+    int s = a.slots[t];
+    if constexpr (ROPE != kNoRope) {
+      const int p = a.positions[t];
+      s = p >= 0 && p < a.max_positions ? s : -1;
+    }
+    return s >= 0 && s / a.block_size < a.num_blocks ? s : -1;
+  };
+  const int slot = slot_of(t0 + lane), before = slot_of(t0 + lane - 1);
+  const bool next = slot >= 0 && before >= 0 && before + 1 == slot && slot % a.group != 0;
+  const uint64_t valid = __builtin_amdgcn_ballot_w64(slot >= 0);
+  const uint64_t lead = valid & ~__builtin_amdgcn_ballot_w64(next);
+  constexpr uint64_t kIn = (1ull << kTileTokens) - 1;
+  if ((lead & kIn) == 0) return;
+  const int lo = __builtin_ctzll(lead & kIn);
+  // the tile's last segment ends before the first token past the tile that leads or is not written
+  const uint64_t stop = (lead | ~valid) & ~kIn;
+  const int hi = stop ? __builtin_ctzll(stop) : kWave;
+  const uint64_t mine = valid & (~0ull << lo) & (hi < kWave ? (1ull << hi) - 1 : ~0ull);
+  // chunks: C tokens of one segment from an aligned slot on
+  uint64_t full = mine & __builtin_amdgcn_ballot_w64(slot % C == 0);
+  const uint64_t follow = mine & ~lead;
+#pragma unroll
+  for (int i = 1; i < C; ++i) full &= follow >> i;
+  uint64_t single = mine;
+#pragma unroll
+  for (int i = 0; i < C; ++i) single &= ~(full << i);
+
+  // the tokens' rows into LDS, in the pool's type
+  const int stride = a.head_size * E + kTileRowPad;
+  const void* src = is_v ? a.value : a.key;
+  auto row_of = [&](int i) { return ((int64_t)(t0 + i) * a.num_kv_heads + h) * a.head_size; };
+  if (ROPE != kNoRope && !is_v) {
+    if constexpr (ROPE != kNoRope) {
+      const int half = a.head_size / 2, units = half / 8;
+      for (int j = tid; j < (hi - lo) * units; j += kTileThreads) {
+        const int i = lo + j / units, u = j % units;
+        if (!(mine >> i & 1)) continue;
+        const int64_t at = (int64_t)a.positions[t0 + i] * half + 8 * u;
+        float c[8], s[8], x[8], y[8];
+        load8f<Kind::F32>(a.cos_table, at, c);
+        load8f<Kind::F32>(a.sin_table, at, s);
+        load_unit<SRC, ROPE>(src, row_of(i), u, half, x, y);
+        rotate_unit<ROPE>(x, y, c, s);
+        char* r = tile_rows + i * stride;
+        stage8<POOL>(r + (ROPE == 0 ? 16 * u : 8 * u) * E, x);
+        stage8<POOL>(r + (ROPE == 0 ? 16 * u + 8 : half + 8 * u) * E, y);
+      }
+    }
+  } else if constexpr (POOL == Kind::FP8) {
+    const int units = a.head_size / 8;
+    const float mul = is_v ? a.v_mul : a.k_mul;
+    for (int j = tid; j < (hi - lo) * units; j += kTileThreads) {
+      const int i = lo + j / units, u = j % units;
+      if (!(mine >> i & 1)) continue;
+      float x[8];
+      load8<SRC>(src, row_of(i) + 8 * u, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = fp32_result(x[e] * mul);
+      stage8<POOL>(tile_rows + i * stride + 8 * u, x);
+    }
+  } else {
+    const int units = a.head_size / C;                          // 16 bytes, as they are
+    for (int j = tid; j < (hi - lo) * units; j += kTileThreads) {
+      const int i = lo + j / units, u = j % units;
+      if (!(mine >> i & 1)) continue;
+      const u32x4 w = load16((const char*)src + (row_of(i) + u * C) * E);
+      uint2* r = reinterpret_cast<uint2*>(tile_rows + i * stride + 16 * u);
+      r[0] = make_uint2(w.x, w.y);
+      r[1] = make_uint2(w.z, w.w);
+    }
+  }
+  __shared__ int64_t at[kWave];                                 // byte of (token, channel 0) in the pool
+  __shared__ uint8_t heads_of[kWave / C];                       // first token of each chunk
+  __shared__ uint8_t alone[kWave];
+  if (tid < kWave) {
+    const uint64_t below = (1ull << lane) - 1;
+    const int blk = slot / a.block_size;
+    at[lane] = (((int64_t)blk * a.num_kv_heads + h) * a.head_size * a.block_size + (slot - blk * a.block_size)) * E;
+    if (full >> lane & 1) heads_of[__builtin_popcountll(full & below)] = (uint8_t)lane;
+    if (single >> lane & 1) alone[__builtin_popcountll(single & below)] = (uint8_t)lane;
+  }
+  __syncthreads();
+
+  char* pool = is_v ? a.v_cache : a.k_cache;
+  const int nf = __builtin_popcountll(full), ns = __builtin_popcountll(single);
+  const int64_t channel = (int64_t)a.block_size * E;
+  // item j is chunk j % nf of channel j / nf: a store's lanes run along each
+  // block's rows.  The quotient by a product is exact for j nf < 65536 (at
+  // most 128 channels x 15 chunks of 4-byte elements: 28800).
+  const unsigned inv = nf ? 65536u / nf + 1 : 0;
+  for (unsigned j = tid; j < (unsigned)(nf * a.head_size); j += kTileThreads) {
+    const int c = (int)(j * inv >> 16), i = heads_of[j - c * nf];
+    const char* col = tile_rows + i * stride + c * E;
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < C; ++e) {
+      const char* p = col + e * stride;
+      const uint32_t v = E == 1 ? *(const uint8_t*)p : E == 2 ? *(const uint16_t*)p : *(const uint32_t*)p;
+      w[e * E / 4] |= v << (8 * (e * E % 4));
+    }
+    *reinterpret_cast<u32x4*>(pool + at[i] + c * channel) = u32x4{w[0], w[1], w[2], w[3]};
+  }
+  for (int j = tid / kWave; j < ns; j += kTileThreads / kWave) {
+    const int i = alone[j];
+    const char* row = tile_rows + i * stride;
+    char* d = pool + at[i];
+    for (int c = lane; c < a.head_size; c += kWave) {
+      if constexpr (E == 1) *(uint8_t*)(d + c * channel) = ((const uint8_t*)row)[c];
+      else if constexpr (E == 2) *(uint16_t*)(d + c * channel) = ((const uint16_t*)row)[c];
+      else *(uint32_t*)(d + c * channel) = ((const uint32_t*)row)[c];
+    }
+  }
+}
+
 // grid.x = pairs x pools x slices; pool 1 is the second (V) pool of a copy.
 template <bool VEC>
 __global__ __launch_bounds__(256) void block_copy_kernel(BlockCopy c) {
@@ -442,16 +702,66 @@ __global__ void scale_finish_kernel(uint32_t* bits) {
   *reinterpret_cast<float*>(bits) = amax / 448.0f;
 }
 
+// Slots of a segment's group: a block, or its largest power-of-two part of
+// at most 32 slots that holds whole 16-byte chunks.
+int tile_group(int block_size, int elem) {
+  if (block_size <= kTileTokens) return block_size;
+  int g = kTileTokens;
+  while (block_size % g) g /= 2;
+  return g * elem >= 16 ? g : 0;
+}
+
+// Whether append_tiles_kernel takes the call: whole 16-byte chunks in a
+// block, 16-byte aligned rows and tables, and rows that leave LDS for
+// several workgroups (63 rows of 512 bytes: 32 KiB).
+bool tile_shape(const TileAppend& a, int src_elem, int elem, bool rope) {
+  auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  if (!al(a.key) || !al(a.value) || !al(a.k_cache) || !al(a.v_cache)) return false;
+  if (rope && (!al(a.cos_table) || !al(a.sin_table) || !al(a.q) || !al(a.q_out))) return false;
+  return a.block_size * elem % 16 == 0 && tile_group(a.block_size, elem) != 0 && a.head_size * elem <= 512 &&
+         (int64_t)a.head_size * src_elem % 16 == 0 && a.head_size * elem % 8 == 0;
+}
+
+template <Kind SRC, Kind POOL, int ROPE>
+int launch_tiles(TileAppend a, hipStream_t stream) {
+  constexpr int E = KindInfo<POOL>::bytes;
+  a.group = tile_group(a.block_size, E);
+  const int64_t tiles = ((int64_t)a.num_tokens + kTileTokens - 1) / kTileTokens;
+  const int64_t kv = tiles * a.num_kv_heads * 2;
+  int64_t grid = kv;
+  if (ROPE != kNoRope) {
+    const int64_t sets = (a.num_heads + kTileHeadsPerThread - 1) / kTileHeadsPerThread;
+    grid += (a.num_tokens * sets * (a.head_size / 16) + kTileThreads - 1) / kTileThreads;
+  }
+  if (grid > 0x7fffffff) return 3;
+  a.kv_wgs = (int)kv;
+  const size_t lds = (size_t)(kTileTokens + a.group - 1) * (a.head_size * E + kTileRowPad);
+  hipLaunchKernelGGL((append_tiles_kernel<SRC, POOL, ROPE>), dim3((unsigned)grid), dim3(kTileThreads), lds, stream,
+                     a);
+  return hipGetLastError() == hipSuccess ? 0 : 5;
+}
+
 }  // namespace
 
 int launch_reshape_and_cache(const CacheLaunch& a) {
   const int64_t runs_per_tok = (int64_t)a.num_kv_heads * (a.head_size / 8);
   if (a.num_tokens == 0) return 0;
+  TileAppend ta = {};
+  ta.key = a.key; ta.value = a.value; ta.k_cache = (char*)a.k_cache; ta.v_cache = (char*)a.v_cache;
+  ta.slots = a.slot_mapping;
+  ta.num_tokens = a.num_tokens; ta.num_kv_heads = a.num_kv_heads; ta.head_size = a.head_size;
+  ta.block_size = a.block_size; ta.num_blocks = a.num_blocks;
+  const bool prompt = a.num_tokens > kRowAppendMaxTokens;
   if (a.cache_dtype == (int)Kind::FP8) {
     const int64_t total = (int64_t)a.num_tokens * runs_per_tok;
     const dim3 grid((unsigned)((total + 255) / 256));
     const float km = 1.0f / (a.k_scale == 0.f ? 1.f : a.k_scale);
     const float vm = 1.0f / (a.v_scale == 0.f ? 1.f : a.v_scale);
+    ta.k_mul = km; ta.v_mul = vm;
+    if (prompt && tile_shape(ta, 2, 1, false)) {
+      if (a.src_dtype == (int)Kind::F16) return launch_tiles<Kind::F16, Kind::FP8, kNoRope>(ta, a.stream);
+      if (a.src_dtype == (int)Kind::BF16) return launch_tiles<Kind::BF16, Kind::FP8, kNoRope>(ta, a.stream);
+    }
     if (a.src_dtype == (int)Kind::F16)
       hipLaunchKernelGGL(reshape_fp8_kernel<Kind::F16>, grid, dim3(256), 0, a.stream, a.key,
                          a.value, (uint8_t*)a.k_cache, (uint8_t*)a.v_cache, a.slot_mapping,
@@ -464,6 +774,9 @@ int launch_reshape_and_cache(const CacheLaunch& a) {
       return 3;
   } else {
     const int E = (a.cache_dtype == (int)Kind::F32) ? 4 : 2;
+    if (prompt && tile_shape(ta, E, E, false))
+      return E == 4 ? launch_tiles<Kind::F32, Kind::F32, kNoRope>(ta, a.stream)
+                    : launch_tiles<Kind::F16, Kind::F16, kNoRope>(ta, a.stream);   // 2-byte copies
     const int64_t total = (int64_t)a.num_tokens * a.num_kv_heads * (a.head_size / (16 / E));
     const dim3 grid((unsigned)((total + 255) / 256));
     const bool aligned = (((uintptr_t)a.k_cache | (uintptr_t)a.v_cache) % 16) == 0;
@@ -503,6 +816,27 @@ int launch_rope_cache(const RopeCache& a_in, hipStream_t stream) {
   // decode-sized calls: one wavefront per (token, kv head), whole block rows
   const bool rows = a.num_tokens <= kRowAppendMaxTokens && (a.block_size * E) % 16 == 0 && aligned &&
                     a.num_heads % a.num_kv_heads == 0;
+  if (a.num_tokens > kRowAppendMaxTokens) {
+    TileAppend ta = {};
+    ta.q = a.q; ta.q_out = a.q_out; ta.key = a.key; ta.value = a.value;
+    ta.k_cache = (char*)a.k_cache; ta.v_cache = (char*)a.v_cache;
+    ta.slots = a.slot_mapping; ta.positions = a.positions;
+    ta.cos_table = a.cos_table; ta.sin_table = a.sin_table;
+    ta.num_tokens = a.num_tokens; ta.num_heads = a.num_heads; ta.num_kv_heads = a.num_kv_heads;
+    ta.head_size = a.head_size; ta.block_size = a.block_size; ta.num_blocks = a.num_blocks;
+    ta.max_positions = a.max_positions;
+    if (tile_shape(ta, E, E, true)) {
+      if (k == Kind::F16)
+        return a.style ? launch_tiles<Kind::F16, Kind::F16, 1>(ta, stream)
+                       : launch_tiles<Kind::F16, Kind::F16, 0>(ta, stream);
+      if (k == Kind::BF16)
+        return a.style ? launch_tiles<Kind::BF16, Kind::BF16, 1>(ta, stream)
+                       : launch_tiles<Kind::BF16, Kind::BF16, 0>(ta, stream);
+      if (k == Kind::F32)
+        return a.style ? launch_tiles<Kind::F32, Kind::F32, 1>(ta, stream)
+                       : launch_tiles<Kind::F32, Kind::F32, 0>(ta, stream);
+    }
+  }
   const int64_t total = (int64_t)a.num_tokens * (a.num_heads + 2 * a.num_kv_heads) * (a.head_size / 16);
   const dim3 grid((unsigned)((total + 255) / 256));
   const dim3 rgrid((unsigned)(a.num_tokens * a.num_kv_heads));
