@@ -207,6 +207,38 @@ def test_build_pages_bit_exact(R, bits):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("BS", [8, 16, 64, 256])
+def test_build_pages_special_values_bit_exact(BS, bits):
+    """Groups whose scan order shows (signed zeros, NaN, infinities), constant and subnormal groups, the largest
+    halves and values midway between two codes, in pages of ordinary ones."""
+    kc = KiviCase(67, [1300, 97, 700, 64], R=32, bits=bits, BS=BS)
+    rng = np.random.default_rng(BS + bits)
+    f16 = lambda *v: np.array(v, np.float16).view(np.uint16)
+    kinds = [f16(0.0, -0.0), f16(np.nan, 1.5, -2.0), f16(np.inf, 3.0), f16(-np.inf, 1.0), f16(np.inf),
+             f16(-np.inf, np.inf, np.nan), f16(2.5), f16(-0.0), f16(6e-8, 0.0, -1.2e-7), f16(65504, -65504, 11),
+             f16(*np.arange(0, 31) / 2), f16(*(np.arange(0, 511, 7) / 2)), f16(np.nan), f16(-0.0, 1.0, 0.0),
+             np.array([0x7C01, 0x3C00, 0xFC01, 0x0001], np.uint16)]   # signalling NaN beside a subnormal
+    N = kc.k.shape[0]
+    for pool in (kc.k, kc.v):
+        for b in rng.choice(N, size=max(1, N // 3), replace=False):
+            for h in range(kc.n_kv):
+                v = kinds[rng.integers(len(kinds))]
+                c0, t0 = 32 * rng.integers(0, 4), rng.integers(0, BS)
+                if rng.random() < 0.5:                   # whole tokens over a group of channels
+                    pool[b, h, c0:c0 + 32, t0] = rng.choice(v, 32)
+                else:                                    # whole channels over the block's tokens
+                    pool[b, h, c0:c0 + 8, :] = rng.choice(v, (8, BS))
+    want = kc.oracle_pages()
+    qd, kd, vd = dev(kc.q, orc.F16), dev(kc.k, orc.F16), dev(kc.v, orc.F16)
+    btd, sld, ptd = dev(kc.tables), dev(kc.lens), dev(kc.page_tables)
+    pages = torch.zeros(kc.num_pages, kc.n_kv, kc.page_bytes, dtype=torch.uint8, device="cuda")
+    print(f"case build pages special values BS={BS} bits={bits}", flush=True)
+    tla.kivi_build_pages(kc.desc(qd, kd, btd, ptd), kd, vd, btd, sld, ptd, pages, int(kc.lens.max()))
+    torch.cuda.synchronize()
+    assert np.array_equal(pages.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 def test_append_quantises_on_page_boundaries(bits):
     """Append one token per step for 70 steps; pages and the fp16 pool match
     a rebuild from the final pool, and pages appear exactly when Lq grows."""

@@ -306,56 +306,341 @@ __global__ __launch_bounds__(kWave) void kivi_vec_decompress_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Paged KIVI: build one page (32 tokens x 128 channels of one kv head) from
-// the fp16 pool [N, n_kv, 128, BS].
+// Paged KIVI append: the new token of each (sequence, kv head) into the fp16
+// pool [N, n_kv, 128, BS], and the page (32 tokens x 128 channels) that it
+// completes, or, with build-ahead, its piece of the next page.
 // ---------------------------------------------------------------------------
 template <int BITS>
-__global__ __launch_bounds__(128) void kivi_page_kernel(PageJob j) {
+__global__ __launch_bounds__(128) void kivi_append_kernel(PageJob j) {
   __shared__ __attribute__((aligned(16))) KiviBuildSmem<BITS> sm;
   const int tid = threadIdx.x;
-  int bid = blockIdx.x;
-  const int kvh = bid % j.num_kv_heads; bid /= j.num_kv_heads;
-  const int pg = bid % j.pages_per_seq_grid;
-  const int seq = bid / j.pages_per_seq_grid;
+  const int kvh = blockIdx.x % j.num_kv_heads, seq = blockIdx.x / j.num_kv_heads;
   const int L = j.seq_lens[seq];
   const int lq = kivi_quantized_len(L, j.residual_length);
-  int page;
+  kivi_append_token<128>(j, seq, kvh, tid);
+  if (j.build_ahead) {
+    // the pages this append completes were written in pieces by the
+    // appends before it; this one writes its piece of the next page:
+    // wavefront 0 stages its fp16, then each wavefront quantises two of
+    // its quarters
+    int ahead_page;
+    const int piece = kivi_ahead_piece(L, j.residual_length, ahead_page);
+    if (piece < 0) return;
+    __shared__ int s_pid;
+    uint16_t* raw = reinterpret_cast<uint16_t*>(&sm.qk[0][0]);
+    const int lane = tid % kWave, wave = tid / kWave;
+    if (wave == 0) {
+      KiviPiece pc = kivi_piece_plan(j, seq, ahead_page, piece, lane);
+      kivi_piece_load(j, pc, kvh, ahead_page, lane);
+      kivi_piece_stage(pc, lane, raw);
+      if (lane == 0) s_pid = pc.piece >= 0 ? pc.pid : -1;
+    }
+    __syncthreads();
+    const int pid = s_pid;
+    if (pid < 0) return;
+    for (int q = wave; q < 4; q += 128 / kWave)
+      kivi_piece_quarter<BITS>(j, pid, piece, kvh, q, lane, kivi_piece_quarter_values(piece, q, lane, raw),
+                               &sm.qv[0][0] + 256 * q);
+    return;
+  }
+  if (lq == 0 || lq == kivi_quantized_len(L - 1, j.residual_length)) return;
+  kivi_build_page<128, BITS>(sm, j, seq, kvh, lq / kKiviPageTokens - 1, L, tid);
+}
+
+// ---------------------------------------------------------------------------
+// Prefix build: every page of a prefix, one workgroup of two wavefronts per
+// (page, kv head), one on K and one on V, with the values in registers.
+//
+// kivi_build_page above gives one thread one group of 32 values that it reads
+// from LDS, and runs each value through some 16 VALU instructions and four
+// LDS accesses of a byte or two; that, and 30 KiB of LDS per workgroup, took
+// 80 us for a build whose bytes need 26.  Here a value costs about 5: min and
+// max over packed halves three at a time, x - min straight from the half
+// (v_fma_mix), one multiply, the rounding as an addition of 2^23 and one
+// shift-add into the packed codes; codes reach their page dwords by exchanges
+// between lanes of a quad or octet.  The page's bytes are kivi_build_page's.
+//
+// 8 prompts of 4096 tokens, 8 kv heads, INT4 (171 MB): 37.9 us = 4.5 TB/s
+// (79.9 before).  Held to fewer registers for 5 or 6 wavefronts per SIMD (116
+// here, 4) it spills: 46 and 54 us.
+// ---------------------------------------------------------------------------
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+
+// Least and greatest of packed halves, element by element; a NaN stays.
+__device__ __forceinline__ half2v pk_min(half2v a, half2v b) { return __builtin_elementwise_minimum(a, b); }
+__device__ __forceinline__ half2v pk_max(half2v a, half2v b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ half2v as_half2(uint32_t w) { return __builtin_bit_cast(half2v, w); }
+
+// The scans of group_params' caller start from +-FLT_MAX, skip NaN and keep
+// the first of equal values.  Over finite values that is the plain least and
+// greatest value, but for the sign of a zero minimum: such groups, and those
+// with a NaN or an infinity, are scanned in order.
+__device__ __forceinline__ bool scan_in_order(float mn, float mx) {
+  return !(mn > -FLT_MAX && mx < FLT_MAX) || mn == 0.0f;
+}
+
+// The codes of quantise over a group of finite values, before packing: the
+// code plus kCodeBias.  x - min is exact in one rounding from the half, the
+// product is rounded by itself (no contraction), and it lies in [0, LEVELS]
+// up to a rounding, so adding 2^23 leaves its nearest-even integer in the low
+// mantissa bits and no clamp is needed.
+constexpr uint32_t kCodeBias = 0x4B000000u;                      // 2^23 in fp32
+__device__ __forceinline__ uint32_t biased_code(_Float16 x, float one, float gmin, float scale) {
+#pragma clang fp contract(off)
+  const float d = __builtin_fmaf((float)x, one, -gmin);
+  const float p = d * scale;
+  return __float_as_uint(p + 8388608.0f);
+}
+
+// N codes of BITS each (8 of 4 bits, 4 of 8) into a dword, code i at bit
+// shift_of(i).
+template <int BITS, int N, bool IN_ORDER, class Value, class Group, class Shift>
+__device__ __forceinline__ uint32_t pack_codes(float one, Value value, Group group, Shift shift_of) {
+  uint32_t acc = 0;
+  if constexpr (IN_ORDER) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      acc |= (uint32_t)quantise<KiviFmt<BITS>::kLevels>((float)value(i), group(i)) << shift_of(i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc -= kCodeBias << shift_of(i);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      acc += biased_code(value(i), one, group(i).gmin, group(i).scale) << shift_of(i);
+  }
+  return acc;
+}
+
+// Exchanges with lane ^ M of one bit of the element position in a dword: the
+// upper of each pair of 16-bit halves, bytes or nibbles goes to the lane with
+// bit M clear, the lower one to the other.
+template <int M>
+__device__ __forceinline__ uint32_t swap_halves(uint32_t own, bool up) {
+  return __builtin_amdgcn_perm(own, lane_xor_u<M>(own), up ? 0x07060302u : 0x01000504u);
+}
+template <int M>
+__device__ __forceinline__ uint32_t swap_bytes(uint32_t own, bool up) {
+  return __builtin_amdgcn_perm(own, lane_xor_u<M>(own), up ? 0x07030501u : 0x02060004u);
+}
+template <int M>
+__device__ __forceinline__ uint32_t swap_nibbles(uint32_t own, bool up) {
+  const uint32_t o = lane_xor_u<M>(own), mask = up ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
+  return (own & mask) | (__builtin_amdgcn_alignbit(o, o, up ? 4 : 28) & ~mask);
+}
+
+// The block of token `tok` of a sequence, or -1.
+__device__ __forceinline__ int block_of_token(const PageJob& j, const int32_t* btab, int tok) {
+  const int lb = tok / j.block_size;
+  const int phys = lb < j.max_blocks_per_seq ? btab[lb] : -1;
+  return phys < 0 || phys >= j.num_blocks ? -1 : phys;
+}
+__device__ __forceinline__ const uint16_t* pool_at(const PageJob& j, const uint16_t* pool, int phys, int kvh, int c,
+                                                   int tok) {
+  return pool + (((int64_t)phys * j.num_kv_heads + kvh) * kKiviHead + c) * j.block_size + tok % j.block_size;
+}
+
+// K of a page.  Lane (tt, jj, ci) = (lane / 32, lane / 8 % 4, lane % 8) takes
+// tokens 16 tt .. 16 tt + 15 of channels 8 (jj + 4 m) + ci, m = 0 .. 3: the
+// channels of one chunk position, whose codes of 8 tokens the lanes of an
+// octet exchange for 8 channels of a token each.
+template <int BITS>
+__device__ __forceinline__ void build_page_k(const PageJob& j, const int32_t* btab, int kvh, int page, uint8_t* dst,
+                                             uint32_t* stage, int lane) {
+  using F = KiviFmt<BITS>;
+  constexpr int LV = F::kLevels, PER = 32 / BITS, DW = 16 / PER;   // codes of a dword, dwords of 16 tokens
+  const int tt = lane >> 5, jj = lane >> 3 & 3, ci = lane & 7;
+  const int tok = page * kKiviPageTokens + 16 * tt;
+  const int phys[2] = {block_of_token(j, btab, tok), block_of_token(j, btab, tok + 8)};
+  uint32_t x[4][8];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const u32x4 v = load16(pool_at(j, j.k_cache, max(phys[r], 0), kvh, 32 * m + 8 * jj + ci, tok + 8 * r));
+      x[m][4 * r] = v.x; x[m][4 * r + 1] = v.y; x[m][4 * r + 2] = v.z; x[m][4 * r + 3] = v.w;
+    }
+  if (__builtin_amdgcn_ballot_w64(phys[0] < 0 || phys[1] < 0)) {  // a block table hole reads as zeros
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[m][i] = phys[i / 4] < 0 ? 0u : x[m][i];
+  }
+  float one = 1.0f;
+  asm volatile("" : "+s"(one));                                  // x - min as one v_fma_mix
+  uint32_t out[4][DW];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    auto value = [&](int i) { return as_half2(x[m][i / 2])[i & 1]; };
+    half2v a = as_half2(x[m][0]), b = a;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      a = pk_min(a, as_half2(x[m][i]));
+      b = pk_max(b, as_half2(x[m][i]));
+    }
+    // the token halves of the channel sit 32 lanes apart
+    a = pk_min(a, as_half2(lane_xor_u<32>(__builtin_bit_cast(uint32_t, a))));
+    b = pk_max(b, as_half2(lane_xor_u<32>(__builtin_bit_cast(uint32_t, b))));
+    float mn = (float)__builtin_elementwise_minimum(a.x, a.y), mx = (float)__builtin_elementwise_maximum(b.x, b.y);
+    const bool in_order = __builtin_amdgcn_ballot_w64(scan_in_order(mn, mx)) != 0;
+    if (in_order) {
+      mn = FLT_MAX;
+      mx = -FLT_MAX;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float v = (float)value(i);
+        if (v < mn) mn = v;
+        if (v > mx) mx = v;
+      }
+      scan_combine_lanes<32, 32>(mn, mx, lane);
+    }
+    const GroupQ g = group_params<LV>(mn, mx);
+    reinterpret_cast<uint16_t*>(dst + F::kKParams + (jj + 4 * m) * 32)[8 * tt + ci] = tt ? g.zero : g.step;
+    // token e of a dword where channel e belongs in the page's
+    auto shift = [&](int e) { return BITS == 4 ? 16 * (e & 1) + 4 * (e >> 1) : 8 * (e >> 1) + 16 * (e & 1); };
+    auto group = [&](int) -> const GroupQ& { return g; };
+#pragma unroll
+    for (int k = 0; k < DW; ++k) {
+      auto val = [&](int e) { return value(PER * k + e); };
+      uint32_t w = in_order ? pack_codes<BITS, PER, true>(one, val, group, shift)
+                            : pack_codes<BITS, PER, false>(one, val, group, shift);
+      w = swap_halves<1>(w, lane & 1);
+      if constexpr (BITS == 4) {
+        w = swap_nibbles<2>(w, lane & 2);
+        w = swap_bytes<4>(w, lane & 4);
+      } else {
+        w = swap_bytes<2>(w, lane & 2);
+      }
+      out[m][k] = w;
+    }
+  }
+  if constexpr (BITS == 4) {
+    // dwords m = 0 .. 3 of tokens 16 tt + 8 k + ci: whole chunks
+#pragma unroll
+    for (int k = 0; k < DW; ++k)
+      reinterpret_cast<u32x4*>(dst + F::kKCodes)[64 * tt + 16 * jj + 8 * k + ci] =
+          u32x4{out[0][k], out[1][k], out[2][k], out[3][k]};
+  } else {
+    // dword 2 m + ci / 4 of tokens 16 tt + 4 k + ci % 4
+#pragma unroll
+    for (int k = 0; k < DW; ++k)
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        stage[(64 * tt + 16 * jj + 4 * k + (ci & 3)) * 8 + 2 * m + (ci >> 2)] = out[m][k];
+    build_barrier<kWave>();
+#pragma unroll
+    for (int i = 0; i < F::kChunk * 2; i += 16)                  // 128 chunks of kChunk bytes, 16 per lane and step
+      reinterpret_cast<u32x4*>(dst + F::kKCodes)[i * 4 + lane] = reinterpret_cast<const u32x4*>(stage)[i * 4 + lane];
+  }
+}
+
+// V of a page.  Lane (g, r, p) = (lane / 16, lane / 4 % 4, lane % 4) takes
+// the two tokens of slots 2 p, 2 p + 1 of lane group r over the 32 channels
+// of group g, so a (token, group)'s least and greatest value need no other
+// lane; the lanes of a quad exchange their tokens' codes of four channels (a
+// pair, of two) for eight (four) slots of one.
+template <int BITS>
+__device__ __forceinline__ void build_page_v(const PageJob& j, const int32_t* btab, int kvh, int page, uint8_t* dst,
+                                             uint32_t* stage, int lane) {
+  using F = KiviFmt<BITS>;
+  constexpr int LV = F::kLevels, CH = 16 / BITS;                 // channels of a packed dword
+  const int g = lane >> 4, r = lane >> 2 & 3, p = lane & 3;
+  const int tok = page * kKiviPageTokens + kivi_v_token(r, 2 * p);
+  const int phys = block_of_token(j, btab, tok);
+  const uint16_t* at = pool_at(j, j.v_cache, max(phys, 0), kvh, 32 * g, tok);
+  uint32_t x[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) x[i] = *reinterpret_cast<const uint32_t*>(at + i * j.block_size);
+  if (__builtin_amdgcn_ballot_w64(phys < 0)) {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) x[i] = phys < 0 ? 0u : x[i];
+  }
+  half2v a = as_half2(x[0]), b = a;
+#pragma unroll
+  for (int i = 1; i < 32; ++i) {
+    a = pk_min(a, as_half2(x[i]));
+    b = pk_max(b, as_half2(x[i]));
+  }
+  float mn[2] = {(float)a.x, (float)a.y}, mx[2] = {(float)b.x, (float)b.y};
+  const bool in_order =
+      __builtin_amdgcn_ballot_w64(scan_in_order(mn[0], mx[0]) || scan_in_order(mn[1], mx[1])) != 0;
+  if (in_order) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      mn[e] = FLT_MAX;
+      mx[e] = -FLT_MAX;
+#pragma unroll
+      for (int i = 0; i < 32; ++i) {
+        const float v = (float)as_half2(x[i])[e];
+        if (v < mn[e]) mn[e] = v;
+        if (v > mx[e]) mx[e] = v;
+      }
+    }
+  }
+  const GroupQ q[2] = {group_params<LV>(mn[0], mx[0]), group_params<LV>(mn[1], mx[1])};
+  uint32_t* params = reinterpret_cast<uint32_t*>(dst + F::kVParams + (4 * g + r) * 32);
+  params[p] = q[0].step | (uint32_t)q[1].step << 16;
+  params[4 + p] = q[0].zero | (uint32_t)q[1].zero << 16;
+
+  float one = 1.0f;
+  asm volatile("" : "+s"(one));
+  // chunks of the stage are permuted (by 4 r or 2 r) against bank conflicts
+  // between the lane groups
+  constexpr int SW = BITS == 4 ? 4 : 2, CD = F::kChunk / 4;
+  auto chunk = [&](int c) { return (64 * (g >> 1) + 16 * r + ((c & 15) ^ (SW * r))) * CD; };
+  // code e of a dword: channel e / 2 of its CH, token e % 2; the second
+  // token in the upper half
+  auto shift = [&](int e) { return 16 * (e & 1) + BITS * (e >> 1); };
+  auto group = [&](int e) -> const GroupQ& { return q[e & 1]; };
+#pragma unroll
+  for (int k = 0; k < 32 / CH; ++k) {
+    auto val = [&](int e) { return as_half2(x[CH * k + (e >> 1)])[e & 1]; };
+    uint32_t w = in_order ? pack_codes<BITS, 2 * CH, true>(one, val, group, shift)
+                          : pack_codes<BITS, 2 * CH, false>(one, val, group, shift);
+    if constexpr (BITS == 4) {
+      w = swap_nibbles<1>(w, lane & 1);
+      w = swap_bytes<2>(w, lane & 2);
+      const int c = 4 * k + p;                                   // of the group's 32
+      stage[chunk(c) + 2 * (g & 1) + (c >> 4)] = w;
+    } else {
+      w = swap_bytes<1>(w, lane & 1);
+      const int c = 2 * k + (p & 1);
+      stage[chunk(c) + 4 * (g & 1) + 2 * (c >> 4) + (p >> 1)] = w;
+    }
+  }
+  build_barrier<kWave>();
+#pragma unroll
+  for (int i = 0; i < F::kChunk * 2; i += 16) {
+    const int at16 = i * 4 + lane, c = at16 / (CD / 4);          // 16 bytes of chunk c
+    const int from = (c ^ (SW * (c >> 4 & 3))) * (CD / 4) + at16 % (CD / 4);
+    reinterpret_cast<u32x4*>(dst + F::kVCodes)[at16] = reinterpret_cast<const u32x4*>(stage)[from];
+  }
+}
+
+template <int BITS>
+__global__ __launch_bounds__(2 * kWave) void kivi_prefix_kernel(PageJob j) {
+  using F = KiviFmt<BITS>;
+  __shared__ __attribute__((aligned(16))) uint32_t stage[2][128 * F::kChunk / 4];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  int bid = blockIdx.x;
+  const int kvh = bid % j.num_kv_heads; bid /= j.num_kv_heads;
+  const int page = bid % j.pages_per_seq_grid;
+  const int seq = bid / j.pages_per_seq_grid;
+  const int L = j.seq_lens[seq];
+  // build-ahead: the next page too once its first piece is due (every piece
+  // written so far and the rest ahead of time: the same bytes)
   int ahead_page;
   const int piece = j.build_ahead ? kivi_ahead_piece(L, j.residual_length, ahead_page) : -1;
-  if (j.append) {
-    kivi_append_token<128>(j, seq, kvh, tid);
-    if (j.build_ahead) {
-      // the pages this append completes were written in pieces by the
-      // appends before it; this one writes its piece of the next page:
-      // wavefront 0 stages its fp16, then each wavefront quantises two of
-      // its quarters
-      if (piece < 0) return;
-      __shared__ int s_pid;
-      uint16_t* raw = reinterpret_cast<uint16_t*>(&sm.qk[0][0]);
-      const int lane = tid % kWave, wave = tid / kWave;
-      if (wave == 0) {
-        KiviPiece pc = kivi_piece_plan(j, seq, ahead_page, piece, lane);
-        kivi_piece_load(j, pc, kvh, ahead_page, lane);
-        kivi_piece_stage(pc, lane, raw);
-        if (lane == 0) s_pid = pc.piece >= 0 ? pc.pid : -1;
-      }
-      __syncthreads();
-      const int pid = s_pid;
-      if (pid < 0) return;
-      for (int q = wave; q < 4; q += 128 / kWave)
-        kivi_piece_quarter<BITS>(j, pid, piece, kvh, q, lane, kivi_piece_quarter_values(piece, q, lane, raw),
-                                 &sm.qv[0][0] + 256 * q);
-      return;
-    }
-    if (lq == 0 || lq == kivi_quantized_len(L - 1, j.residual_length)) return;
-    page = lq / kKiviPageTokens - 1;
-  } else {
-    page = pg;
-    // build-ahead: the next page too once its first piece is due (every
-    // piece written so far and the rest ahead of time: the same bytes)
-    if (page >= lq / kKiviPageTokens && !(piece >= 0 && page == ahead_page)) return;
-  }
-  kivi_build_page<128, BITS>(sm, j, seq, kvh, page, L, tid);
+  if (page >= kivi_quantized_len(L, j.residual_length) / kKiviPageTokens && !(piece >= 0 && page == ahead_page)) return;
+  if (page >= j.max_pages_per_seq) return;
+  const int pid = j.page_tables[(int64_t)seq * j.max_pages_per_seq + page];
+  if (pid < 0 || pid >= j.num_pages) return;
+  uint8_t* dst = j.pages + ((int64_t)pid * j.num_kv_heads + kvh) * F::kBytes;
+  const int32_t* btab = j.block_tables + (int64_t)seq * j.max_blocks_per_seq;
+  if (wave == 0)
+    build_page_k<BITS>(j, btab, kvh, page, dst, stage[0], lane);
+  else
+    build_page_v<BITS>(j, btab, kvh, page, dst, stage[1], lane);
 }
 
 }  // namespace
@@ -389,10 +674,12 @@ int launch_kivi_pages(const KiviPageLaunch& a) {
   if (!a.append && a.max_pages_to_build <= 0) return 0;
   const PageJob j = make_page_job(a);
   const dim3 grid((unsigned)(a.num_seqs * j.pages_per_seq_grid * a.num_kv_heads));
-  if (a.bits == 8)
-    hipLaunchKernelGGL(kivi_page_kernel<8>, grid, dim3(128), 0, a.stream, j);
-  else
-    hipLaunchKernelGGL(kivi_page_kernel<4>, grid, dim3(128), 0, a.stream, j);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(128), 0, a.stream, j); };
+  if (a.append) {
+    if (a.bits == 8) go(kivi_append_kernel<8>); else go(kivi_append_kernel<4>);
+  } else {
+    if (a.bits == 8) go(kivi_prefix_kernel<8>); else go(kivi_prefix_kernel<4>);
+  }
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
 
