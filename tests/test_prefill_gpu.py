@@ -325,3 +325,30 @@ def test_fp8_pool_group_sizes_and_head_maps(gqa):
                                        orc.BF16, 16)
         print(f"case prefill fp8 H={H} n_kv={n_kv} gqa={gqa}", flush=True)
         assert_close(_run_fp8(pc, k8, v8, ks, vs, gqa), _ref_fp8(pc, gqa), orc.BF16, 1e-2, f"fp8 H={H}")
+
+
+@pytest.mark.parametrize("H,n_kv", [(16, 4), (4, 4), (24, 2)])
+@pytest.mark.parametrize("BS", [8, 16, 64, 256])
+@pytest.mark.parametrize("kv", ["bf16", "f16", "fp8"])
+def test_few_and_many_tiles_match_oracle(kv, BS, H, n_kv):
+    """The same prompts as a call of few row tiles (its decode rows not counted as prompts: keys split over a
+    workgroup's wavefronts) and of many.  Lengths end on, before and past an iteration of 64 keys and a round of
+    four of them; rows end inside a 32-row wavefront and a 64-row tile; holes in the tables."""
+    shape = [(2, 2), (21, 63), (64, 64), (17, 65), (9, 256), (100, 513)] + [(1, 40 + 9 * i) for i in range(20)]
+    code = orc.F16 if kv == "f16" else orc.BF16
+    if kv == "fp8":
+        pc, k8, v8, ks, vs = _fp8_case(inputs.SEEDS[4] + BS, shape, H, n_kv, code, BS, holes=3)
+        want, extra = _ref_fp8(pc), dict(kv_dtype=tla.FP8_E4M3, k_scale=ks, v_scale=vs)
+        k, v = torch.from_numpy(k8).cuda(), torch.from_numpy(v8).cuda()
+    else:
+        pc = PrefillCase(inputs.SEEDS[4] + BS, shape, H, n_kv, code, BS=BS, holes=3, nan_unused=True)
+        want, extra = pc.ref(), {}
+        k, v = dev(pc.case.k_cache, code), dev(pc.case.v_cache, code)
+    q, bt, sl, cu = dev(pc.q, code), dev(pc.case.tables), dev(pc.lens), dev(pc.cu)
+    for prompts in (6, 0):
+        out = torch.full_like(q, float("nan"))
+        desc = tla.make_prefill_desc(q, k, bt, pc.S, n_kv, pc.case.scale, num_prefill_seqs=prompts, **extra)
+        print(f"case prefill tiles {kv} BS={BS} H={H} n_kv={n_kv} prompts={prompts}", flush=True)
+        tla.chunked_prefill(desc, out, q, cu, k, v, bt, sl, int(pc.q_lens.max()))
+        torch.cuda.synchronize()
+        assert_close(out, want, code, 1e-2 if kv == "fp8" else ATOL, f"prompts={prompts}")

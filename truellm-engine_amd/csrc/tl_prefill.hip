@@ -129,6 +129,7 @@ struct PrefillParams {
   int num_seqs, row_tiles;
   int pf_seqs;                 // sequences [0, pf_seqs) may be prefill rows
   int dec_first;               // sequences [dec_first, num_seqs) may be decode rows
+  int split;                   // prefill tiles: prefill_split_kernel
 };
 
 template <int NW>
@@ -749,6 +750,404 @@ __global__ __launch_bounds__(NW * kWave) void prefill_kernel(PrefillParams pp) {
   }
 }
 
+// ---- few tiles: keys split over the wavefronts of a workgroup ----
+//
+// prefill_kernel gives a workgroup 256 rows and all their keys: one user's
+// chunk of 500 queries x 4 heads is 8 tiles per kv head, 64 workgroups for
+// 256 CUs, each alone with its serial walk over the keys.  Here a workgroup
+// takes kSplitRows rows: two wavefronts of 32 rows for each of kSplit key
+// groups, group k with iterations k, k + kSplit, ..., each group with a K and
+// a V stage of its own, and the groups' outputs merged through LDS at the
+// end (max, sum, rescaled partial outputs in fp32, summed in group order).
+// Four times the tiles and a quarter of the walk; each key's K and V are
+// read by four times the workgroups, from the L2 of the XCD where the
+// launch order puts a kv head's workgroups (n_kv 8).  The stages fill the
+// CU's LDS (one workgroup, two wavefronts per SIMD, which overlap each
+// other's matrix and VALU work without a schedule).
+//
+// Bound by what a CU takes in: an iteration of its four groups is 128 KB from
+// L2 and through LDS for 64 rows (prefill_kernel: 32 KB for 256), so it pays
+// only while the other kernel leaves CUs idle.  f16, 32/8 heads, us, before
+// and after: 500 queries of 1500 keys 52.4 and 26.5; bf16: 256 of 256 17.0
+// and 11.0, 512 of 6000 187.6 and 88.6, 16 of 3000 95.7 and 47.7.
+constexpr int kSplit = 4;                    // key groups of a workgroup
+constexpr int kSplitWaves = 2;               // wavefronts (32 rows each) of a key group
+constexpr int kSplitRows = kSplitWaves * kPfRows;
+constexpr int kSplitNW = kSplit * kSplitWaves;
+
+struct PrefillSplitSmem {
+  union {
+    struct {
+      uint16_t kt[kSplit][kPfHead * kKtStride];        // [channel][key] (+16 pad)
+      uint16_t v[kSplit][kPfHead * kVStride];          // [channel][v_slot(key)] (+8 pad)
+    } st;
+    float o[kSplitNW][4][4][kWave][4];                 // [wavefront][channel quarter][row quad][lane][row]
+  };
+  float row[kSplitNW][kPfRows];                        // per-row exchange within a wavefront
+  float m[kSplitNW][kPfRows], l[kSplitNW][kPfRows];
+};
+
+template <Kind Q, Kind KV, int BS>
+__global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(PrefillParams pp) {
+  static_assert(BS >= 8 && BS <= 256 && (BS & (BS - 1)) == 0, "block size: a power of two 8 .. 256");
+  static_assert(KV == Q || KV == Kind::FP8, "a 2-byte pool holds the q type");
+  constexpr int BSE = BS >= kPfKeys ? kPfKeys : BS;       // keys of an iteration per block
+  constexpr int BPI = kPfKeys / BSE;                      // pool blocks per iteration
+  constexpr int NKE = BS == 8 ? 2 : 1;                    // blocks of a 16-key run
+  constexpr int E = KV == Kind::FP8 ? 1 : 2;              // pool bytes per element
+  using M = Mfma32<Q>;                                 // q.k
+  using MP = Mfma32<Kind::F16>;                        // p.v (f16 for every type)
+  __shared__ __attribute__((aligned(16))) PrefillSplitSmem sm;
+
+  const Params& p = pp.base;
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = lane >> 5, c32 = lane & 31;
+  const int grp = wave / kSplitWaves, wr = wave % kSplitWaves;
+
+  int b = blockIdx.x;
+  const int items = pp.pf_seqs * p.num_kv_heads;
+  const int tile = pp.row_tiles - 1 - b / items;       // longest (latest) tiles first
+  b %= items;
+  const int seq = b / p.num_kv_heads, kvh = b % p.num_kv_heads;
+  const int32_t* table = p.block_tables + (int64_t)seq * p.max_blocks_per_seq;
+  // entries of iteration it: lane i (< BPI) holds that of block i
+  auto table_read = [&](int it) {
+    const int lb = (int)((unsigned)(it * kPfKeys + min(lane, BPI - 1) * BSE) / BS);
+    return table[min(lb, p.max_blocks_per_seq - 1)];
+  };
+  // the first two iterations' entries are read with the lengths, before the
+  // exits that depend on them: one memory round trip for all
+  int t_cur = table_read(grp), t_next = table_read(grp + kSplit);
+  const int q0 = pp.cu_q_lens[seq], ql = pp.cu_q_lens[seq + 1] - q0;
+  const int L = p.seq_lens[seq];
+  if (ql <= 1) return;                                 // decode rows: prefill_decode_kernel
+  const int rows = ql * p.group, row0 = tile * kSplitRows;
+  if (row0 >= rows) return;
+  const int wrow0 = row0 + wr * kPfRows, my_row = wrow0 + c32;
+  const bool row_ok = my_row < rows;
+  const int qi = row_ok ? my_row / p.group : 0, gi = row_ok ? my_row % p.group : 0;
+  const int pos = row_ok ? L - ql + qi : -1;           // keys 0 .. pos
+  const int last_row = min(rows, row0 + kSplitRows) - 1;
+  const int kend = __builtin_amdgcn_readfirstlane(max(0, L - ql + last_row / p.group + 1));
+  const int n_it = (kend + kPfKeys - 1) / kPfKeys;
+
+  // physical block of the iteration's keys from kk on, or -1
+  auto block_at = [&](int it, int entries, int kk) {
+    const int e = __builtin_amdgcn_readlane(entries, kk / BSE);
+    return it * kPfKeys + kk < kend ? checked_block(p, (int)((unsigned)(it * kPfKeys + kk) / BS), e) : -1;
+  };
+
+  // Staging: a wavefront copies keys 32 wr .. + 31 of its group's iteration
+  // as units of 16 keys x 32 channels: lane l channel l % 32 of the unit and
+  // 8 keys, so that a load reads 1 KB (FP8: 512 B) contiguous in the pool at
+  // block sizes 16 and 32 (as prefill_kernel's).
+  constexpr int kRuns = kPfKeys / 16 / kSplitWaves, kUnits = 4;
+  struct Fetched { u32x4 k[kRuns][kUnits], v[kRuns][kUnits]; int nv[kRuns]; };
+  const int64_t head_bytes = (int64_t)kPfHead * BS * E;
+  auto rsrc_of = [&](const char* pool, int pb) {
+    const int64_t row = ((int64_t)max(pb, 0) * p.num_kv_heads + kvh) * head_bytes;
+    return buffer_rsrc(pool + row, pb >= 0 ? unsigned(head_bytes) : 0u);
+  };
+  auto load_raw = [&](__amdgpu_buffer_rsrc_t r, unsigned off) -> u32x4 {
+    if constexpr (E == 2) {
+      return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    } else {
+      const auto w = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+      return u32x4{(uint32_t)w[0], (uint32_t)w[1], 0u, 0u};
+    }
+  };
+  auto run_key = [&](int r) { return 16 * (kRuns * wr + r); };
+  // the copy's K (PART 0) or V (1)
+  auto fetch = [&](int it, int entries, Fetched& f, auto part) {
+    constexpr int PART = decltype(part)::value;
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      int pb[NKE];
+#pragma unroll
+      for (int h = 0; h < NKE; ++h) pb[h] = block_at(it, entries, run_key(r) + 8 * h);
+      const int tok = run_key(r) + 8 * g;
+      if constexpr (PART == 1) {
+        const int pb_lane = NKE == 2 ? (g ? pb[NKE - 1] : pb[0]) : pb[0];
+        f.nv[r] = pb_lane >= 0 ? min(max(L - (it * kPfKeys + tok), 0), 8) : 0;
+      }
+      const int in_blk = BS > kPfKeys ? (int)((unsigned)(it * kPfKeys) % BS) + tok : tok % BS;
+#pragma unroll
+      for (int u = 0; u < kUnits; ++u) {
+        const char* pool = PART == 0 ? p.k_cache : p.v_cache;
+        const unsigned off = unsigned(E * ((32 * u + c32) * BS + in_blk));
+        u32x4 w;
+        if constexpr (NKE == 1) {
+          w = load_raw(rsrc_of(pool, pb[0]), off);
+        } else {
+          // each load serves one lane half; the other half's offset lies
+          // past the range (no memory request, zeros)
+          constexpr unsigned kPast = 0x40000000u;
+          const u32x4 a = load_raw(rsrc_of(pool, pb[0]), g == 0 ? off : kPast);
+          const u32x4 c = load_raw(rsrc_of(pool, pb[1]), g == 1 ? off : kPast);
+          w = u32x4{a.x | c.x, a.y | c.y, a.z | c.z, a.w | c.w};
+        }
+        (PART == 0 ? f.k : f.v)[r][u] = w;
+      }
+    }
+  };
+  const std::integral_constant<int, 0> kKeys;
+  const std::integral_constant<int, 1> kValues;
+  auto stage = [&](const Fetched& f) {
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      const int tok = run_key(r) + 8 * g;
+#pragma unroll
+      for (int u = 0; u < kUnits; ++u)
+        *reinterpret_cast<u32x4*>(&sm.st.kt[grp][(32 * u + c32) * kKtStride + tok]) =
+            KV == Kind::FP8 ? fp8x8_to<Q>(f.k[r][u]) : f.k[r][u];
+    }
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      const int tok = run_key(r) + 8 * g;
+#pragma unroll
+      for (int u = 0; u < kUnits; ++u) {
+        const int ch = 32 * u + c32;
+        // V slots at or past the sequence end may hold anything: zero them
+        u4v v = __builtin_bit_cast(u4v, KV == Kind::FP8 ? fp8x8_to<Kind::F16>(f.v[r][u]) : f.v[r][u]);
+        const int nv = f.nv[r];
+        if (__builtin_amdgcn_ballot_w64(nv < 8)) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) v[w] = 2 * w >= nv ? 0u : (2 * w + 1 >= nv ? v[w] & 0xFFFFu : v[w]);
+        }
+        if constexpr (KV == Kind::BF16) {
+          // bf16 -> f16, times 2^-7 (see PvScale)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const unsigned x = (unsigned)v[w];
+            v[w] = MP::pack(__builtin_bit_cast(float, x << 16) * PvScale<KV>::kV,
+                            __builtin_bit_cast(float, x & 0xFFFF0000u) * PvScale<KV>::kV);
+          }
+        }
+        uint16_t* vrow = &sm.st.v[grp][ch * kVStride];
+        *reinterpret_cast<uint2*>(vrow + v_slot(tok)) = uint2{v[0], v[1]};
+        *reinterpret_cast<uint2*>(vrow + v_slot(tok + 4)) = uint2{v[2], v[3]};
+      }
+    }
+  };
+
+  // the first copy and q go out together
+  Fetched f;
+  fetch(grp, t_cur, f, kKeys);
+  fetch(grp, t_cur, f, kValues);
+  u32x4 qb[8];
+  {
+    const uint16_t* qrow = (const uint16_t*)p.q +
+        ((int64_t)(q0 + qi) * p.num_heads + head_of(p, kvh, gi)) * kPfHead + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qb[ks] = load16(qrow + 16 * ks);
+    // waited for here: a first use in the loop waits there in every
+    // iteration, for the copy in flight
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) asm volatile("" ::"v"(__builtin_bit_cast(u4v, qb[ks])));
+  }
+
+  f16v o[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) o[c] = f16v{};
+  float m_used = -INFINITY, l_part = 0.f;
+  float* s_row = &sm.row[wave][0];
+  auto wave_sync = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // O rows of this lane (8 j + 4 g + i) times a per-row factor held at lane c32
+  auto scale_rows = [&](float a_row) {
+    if (g == 0) s_row[c32] = a_row;
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 a4 = *reinterpret_cast<const float4*>(&s_row[8 * j + 4 * g]);
+      const float a[4] = {a4.x, a4.y, a4.z, a4.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[c][4 * j + i] *= a[i];
+    }
+    wave_sync();
+  };
+  const int wmin_pos = __builtin_amdgcn_readfirstlane(L - ql + wrow0 / p.group);
+  const int pos_g = pos - 4 * g;
+
+  auto attend = [&](int it, int entries, auto after_scores) {
+    const int k0 = it * kPfKeys;
+    f16v sp[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) sp[t] = f16v{};
+    // the LDS reads are kept ahead of the matrix ops, as in prefill_kernel
+    constexpr int kAhead = 2;
+    u32x4 kb[kAhead + 1][KT], vb[2][4];
+    auto k_op = [&](int t, int ks) { return k_operand(sm.st.kt[grp], t, ks, lane); };
+    auto v_op = [&](int q, int c) {
+      return *reinterpret_cast<const u32x4*>(&sm.st.v[grp][(32 * c + c32) * kVStride + 16 * q + 8 * g]);
+    };
+#pragma unroll
+    for (int ks = 0; ks < kAhead; ++ks)
+#pragma unroll
+      for (int t = 0; t < KT; ++t) kb[ks][t] = k_op(t, ks);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      if (ks + kAhead < 8) {
+#pragma unroll
+        for (int t = 0; t < KT; ++t) kb[(ks + kAhead) % (kAhead + 1)][t] = k_op(t, ks + kAhead);
+      } else if (ks + kAhead == 8) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) vb[0][c] = v_op(0, c);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < KT; ++t) sp[t] = M::mma(kb[ks % (kAhead + 1)][t], qb[ks], sp[t]);
+    }
+    after_scores();
+    bool blk_ok[BPI], all_ok = k0 + kPfKeys - 1 <= wmin_pos;
+#pragma unroll
+    for (int i = 0; i < BPI; ++i) {
+      blk_ok[i] = checked_block(p, (int)((unsigned)(k0 + i * BSE) / BS), __builtin_amdgcn_readlane(entries, i)) >= 0;
+      all_ok = all_ok && blk_ok[i];
+    }
+    if (!all_ok) {
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kc = 32 * t + 8 * (r >> 2) + (r & 3);         // key k0 + kc + 4 g
+          sp[t][r] = k0 + kc <= pos_g && blk_ok[(kc + 4 * g) / BSE] ? sp[t][r] : -INFINITY;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sp[t][r]);
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx),
+                                                       __builtin_bit_cast(unsigned, mx), false, false);
+      mx = fmaxf(__builtin_bit_cast(float, (unsigned)sw[0]), __builtin_bit_cast(float, (unsigned)sw[1]));
+    }
+    mx *= p.qk_scale;
+    const bool raise = mx > m_used + kLazyRescale || (m_used == -INFINITY && mx != -INFINITY);
+    if (__builtin_amdgcn_ballot_w64(raise)) {
+      const float m_new = raise ? mx : m_used;
+      const float alpha = (m_new == m_used) ? 1.f : (m_used == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_used - m_new));
+      m_used = m_new;
+      l_part *= alpha;
+      scale_rows(alpha);
+    }
+    const float m_use = ((m_used == -INFINITY) ? 0.f : m_used) - (float)PvScale<KV>::kPExp;
+    u32x4 pa[KT][2];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      float pw[16], ls[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        pw[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sp[t][r], p.qk_scale, -m_use));
+        ls[r & 3] += pw[r];
+      }
+      l_part += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+        pa[t][s2] = u32x4{MP::pack(pw[8 * s2], pw[8 * s2 + 1]), MP::pack(pw[8 * s2 + 2], pw[8 * s2 + 3]),
+                          MP::pack(pw[8 * s2 + 4], pw[8 * s2 + 5]), MP::pack(pw[8 * s2 + 6], pw[8 * s2 + 7])};
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q + 1 < 4) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) vb[(q + 1) & 1][c] = v_op(q + 1, c);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] = MP::mma(pa[q >> 1][q & 1], vb[q & 1][c], o[c]);
+    }
+  };
+
+  // Every wavefront passes the same barriers, and every path leaves the same
+  // loads in flight: copies past the last iteration are empty (missing
+  // blocks, no traffic), and a group's iteration past it is all masked.  K's
+  // copy goes out before the scores are formed, V's after, when the
+  // registers of the K operands are free.
+  int it = grp;
+#pragma unroll 1
+  for (int base = 0; base < n_it; base += kSplit, it += kSplit) {
+    if (base > 0) __syncthreads();                     // the stage's last readers are done
+    stage(f);
+    const int t_mask = t_cur;
+    t_cur = t_next;
+    fetch(it + kSplit, t_cur, f, kKeys);
+    t_next = table_read(it + 2 * kSplit);
+    __syncthreads();
+    attend(it, t_mask, [&]() { fetch(it + kSplit, t_cur, f, kValues); });
+  }
+
+  // ---- merge: every group's rows on the common maximum ----
+  {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, l_part),
+                                                     __builtin_bit_cast(unsigned, l_part), false, false);
+    const float l = __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
+    if (g == 0) {
+      sm.m[wave][c32] = m_used;
+      sm.l[wave][c32] = l;
+    }
+  }
+  __syncthreads();                                     // the last stage's readers too
+  float m_all = -INFINITY, l_all = 0.f;
+#pragma unroll
+  for (int k = 0; k < kSplit; ++k) m_all = fmaxf(m_all, sm.m[k * kSplitWaves + wr][c32]);
+  auto factor = [&](float m) { return m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_all); };
+#pragma unroll
+  for (int k = 0; k < kSplit; ++k)
+    l_all = __builtin_fmaf(sm.l[k * kSplitWaves + wr][c32], factor(sm.m[k * kSplitWaves + wr][c32]), l_all);
+  scale_rows(factor(m_used));
+  // group k finishes channel quarter k of the rows
+  static_assert(kSplit == 4, "a channel quarter for each group");
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<float4*>(sm.o[wave][c][j][lane]) =
+          make_float4(o[c][4 * j], o[c][4 * j + 1], o[c][4 * j + 2], o[c][4 * j + 3]);
+  if (g == 0) s_row[c32] = l_all > 0.f ? PvScale<KV>::kP * __builtin_amdgcn_rcpf(l_all) : 0.f;   // the sums carry 2^kPExp
+  __syncthreads();
+
+  const float rg = 1.f / (float)p.group;               // rows of the output as in prefill_kernel
+  const int64_t obase = (int64_t)q0 * p.num_heads + (p.gqa_map ? kvh * p.group : kvh);
+  const int rmul = p.gqa_map ? 1 : p.num_kv_heads, qmul = p.gqa_map ? p.num_heads - p.group : 0;
+  const bool odd = (c32 & 1) != 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kSplit; ++k) {
+      const float4 w = *reinterpret_cast<const float4*>(sm.o[k * kSplitWaves + wr][grp][j][lane]);
+      a[0] += w.x; a[1] += w.y; a[2] += w.z; a[3] += w.w;
+    }
+    const float4 i4 = *reinterpret_cast<const float4*>(&s_row[8 * j + 4 * g]);
+    const float inv[4] = {i4.x, i4.y, i4.z, i4.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[i] *= inv[i];
+      if constexpr (KV == Kind::FP8) a[i] *= p.v_scale;
+    }
+    // two channels per 4-byte store: lanes 2 k and 2 k + 1 swap one value
+#pragma unroll
+    for (int ip = 0; ip < 4; ip += 2) {
+      const int row = wrow0 + 8 * j + 4 * g + ip + (odd ? 1 : 0);
+      const int qr = (int)(((float)row + 0.5f) * rg);
+      const float got = dpp<kDppXor1>(odd ? a[ip] : a[ip + 1]);
+      if (row < rows)
+        *reinterpret_cast<uint32_t*>((uint16_t*)p.out + (obase + (int64_t)row * rmul + (int64_t)qr * qmul) * kPfHead +
+                                     32 * grp + (c32 & ~1)) = odd ? M::pack(got, a[ip + 1]) : M::pack(a[ip], got);
+    }
+  }
+}
+
 // Decode rows (q_len == 1) of a mixed batch, one workgroup per (sequence,
 // kv head, 16-head slice), q / out row cu_q_lens[s]: the matrix-core decode
 // wavefronts (tl_mfma_wave.hpp), so a GQA group of up to 16 heads reads its
@@ -784,7 +1183,9 @@ int launch_prefill_t(const PrefillParams& pp, unsigned grid, hipStream_t stream)
   const unsigned dgrid = (unsigned)((pp.num_seqs - pp.dec_first) * p.num_kv_heads * ((p.group + GT - 1) / GT));
   if (dgrid > 0)
     hipLaunchKernelGGL((prefill_decode_kernel<Q, KV, BS, NWD>), dim3(dgrid), dim3(NWD * kWave), 0, stream, pp);
-  if (grid > 0)
+  if (grid > 0 && pp.split)
+    hipLaunchKernelGGL((prefill_split_kernel<Q, KV, BS>), dim3(grid), dim3(kSplitNW * kWave), 0, stream, pp);
+  else if (grid > 0)
     hipLaunchKernelGGL((prefill_kernel<Q, KV, BS, NW>), dim3(grid), dim3(NW * kWave), 0, stream, pp);
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
@@ -803,6 +1204,14 @@ int launch_prefill_bs(const PrefillParams& pp, int bs, unsigned grid, hipStream_
 }
 
 }  // namespace
+
+// Calls of at most this many 256-row tiles take the split kernel: four times
+// the workgroups, then, still run in one round, one per CU.  Measured against
+// prefill_kernel (bf16, 32/8 heads, us): at 64 tiles, 500 of 1500 keys 29.1
+// against 55.0; past the line, at 128, 2 prompts of 512 of 1500 51.6 against
+// 56.6, 4 of 256 of 1024 41.9 against 40.5, 8 of 128 of 128 21.4 against
+// 14.4, and at 256 tiles 100 against 60.
+constexpr int kSplitMaxTiles = 64;
 
 int launch_prefill(const PrefillLaunch& a) {
   constexpr int NW = 8;
@@ -832,6 +1241,11 @@ int launch_prefill(const PrefillLaunch& a) {
   pp.dec_first = a.num_prefill_seqs > 0 ? a.num_prefill_seqs : 0;
   // prefill tiles exist only for q_len > 1
   pp.row_tiles = a.max_q_len > 1 ? (a.max_q_len * p.group + NW * kPfRows - 1) / (NW * kPfRows) : 0;
+  // (a table of at most 64 keys has one iteration and nothing to split: 16
+  // of 16 keys 9.4 us, 10.9 split)
+  pp.split = (int64_t)pp.row_tiles * pp.pf_seqs * a.num_kv_heads <= kSplitMaxTiles &&
+             (int64_t)a.max_blocks_per_seq * a.block_size > kPfKeys;
+  if (pp.split && pp.row_tiles) pp.row_tiles = (a.max_q_len * p.group + kSplitRows - 1) / kSplitRows;
   const unsigned grid = (unsigned)(pp.row_tiles * pp.pf_seqs * a.num_kv_heads);
   const bool bf16 = a.dtype == (int)Kind::BF16;
   if (fp8)
