@@ -85,6 +85,29 @@ def test_vector_codec_slot_counts_and_alignment(D, O, G, n, skew):
     assert np.array_equal(host_bits(back).ravel(), orc.kivi_decompress(want, n, D, O, G).ravel())
 
 
+@pytest.mark.parametrize("D,O,G", [(128, 8, 16), (128, 1, 16), (96, 13, 8), (128, 24, 4), (128, 64, 16), (40, 7, 6)])
+def test_vector_codec_equal_magnitudes(D, O, G):
+    """Few distinct magnitudes of either sign, with NaN, infinities and zeros between them: which of equal values
+    stays, and in which slot, is the order of the scan; groups of zeros of both signs."""
+    rng = np.random.default_rng(D + O)
+    n = 200
+    few = np.array([0.0, -0.0, 0.5, -0.5, 1.0, -1.0, 1.5, -2.0, 2.0, np.inf, -np.inf, np.nan], np.float16)
+    p = np.array([3, 3, 4, 4, 4, 4, 2, 2, 2, .3, .3, .3])
+    xb = np.ascontiguousarray(rng.choice(few, (n, D), p=p / p.sum()).view(np.uint16))
+    xb[::3] = rng.choice(few[:2], (len(xb[::3]), D)).view(np.uint16)
+    stride = orc.kivi_compressed_bytes(D, O, G)
+    want = np.full(n * stride, 0xAB, np.uint8)
+    orc.kivi_compress(xb, D, O, G, out=want)
+    rec = torch.full((n * stride,), 0xAB, dtype=torch.uint8, device="cuda")
+    print(f"case vec codec ties D={D} O={O} G={G}", flush=True)
+    tla.kivi_compress(dev(xb, orc.F16), rec, n, D, O, G)
+    back = torch.zeros(n, D, dtype=torch.float16, device="cuda")
+    tla.kivi_decompress(rec, back, n, D, O, G)
+    torch.cuda.synchronize()
+    assert np.array_equal(rec.cpu().numpy(), want)
+    assert np.array_equal(host_bits(back).ravel(), orc.kivi_decompress(want, n, D, O, G).ravel())
+
+
 def test_vector_codec_hand_derived_slot_order():
     """The kernel writes the outliers in the reference's selection-slot order
     (kivi_cache.cu:50-78), byte for byte against records derived by hand

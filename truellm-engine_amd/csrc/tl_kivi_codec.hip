@@ -26,6 +26,34 @@ namespace tl {
 
 namespace {
 
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+
+// Least and greatest of packed halves, element by element; a NaN stays.
+__device__ __forceinline__ half2v pk_min(half2v a, half2v b) { return __builtin_elementwise_minimum(a, b); }
+__device__ __forceinline__ half2v pk_max(half2v a, half2v b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ half2v as_half2(uint32_t w) { return __builtin_bit_cast(half2v, w); }
+
+// The scans of group_params' caller start from +-FLT_MAX, skip NaN and keep
+// the first of equal values.  Over finite values that is the plain least and
+// greatest value, but for the sign of a zero minimum: such groups, and those
+// with a NaN or an infinity, are scanned in order.
+__device__ __forceinline__ bool scan_in_order(float mn, float mx) {
+  return !(mn > -FLT_MAX && mx < FLT_MAX) || mn == 0.0f;
+}
+
+// The codes of quantise over a group of finite values, before packing: the
+// code plus kCodeBias.  x - min is exact in one rounding from the half, the
+// product is rounded by itself (no contraction), and it lies in [0, LEVELS]
+// up to a rounding, so adding 2^23 leaves its nearest-even integer in the low
+// mantissa bits and no clamp is needed.
+constexpr uint32_t kCodeBias = 0x4B000000u;                      // 2^23 in fp32
+__device__ __forceinline__ uint32_t biased_code(_Float16 x, float one, float gmin, float scale) {
+#pragma clang fp contract(off)
+  const float d = __builtin_fmaf((float)x, one, -gmin);
+  const float p = d * scale;
+  return __float_as_uint(p + 8388608.0f);
+}
+
 // ---------------------------------------------------------------------------
 // The reference vector codec.  8 lanes share a vector, a 64-thread workgroup
 // takes 8 vectors: 16 384 vectors are 2048 wavefronts, two per SIMD.  The
@@ -33,10 +61,12 @@ namespace {
 // sequential over the channels, but each of its steps is the work of 8
 // lanes; the rest (ranks, groups, codes) is spread over them.  Rows and
 // records go through LDS, so that memory sees whole lines.  Bound: the
-// 128-step scan's dependency chain (about 12 vector instructions a step at
-// up to 8 outliers).  Compress and decompress of 16 384 vectors of 128
-// channels, 8 outliers, groups of 16: 23.9 us; one thread per vector, with
-// its slots, flags and values in scratch memory, took 1488 us (783 + 706).
+// 128-step scan's dependency chain (about 6 vector instructions a step at up
+// to 8 outliers) and the few wavefronts there are to hide the rest.  Compress
+// and decompress of 16 384 vectors of 128 channels, 8 outliers, groups of 16:
+// 16.8 us; with a minimum over the slots in each step, values widened one by
+// one and divisions in the copies 23.8 us; one thread per vector, with its
+// slots, flags and values in scratch memory, 1488 us.
 // ---------------------------------------------------------------------------
 constexpr int kVecLanes = 8, kVecVecs = kWave / kVecLanes;
 constexpr int kVecRow = kKiviMaxHeadDim + 8;          // halves per LDS row (16-byte rows, shifted banks)
@@ -50,37 +80,48 @@ template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
 }
-// Over the 8 lanes of a vector.
-__device__ __forceinline__ uint32_t min8(uint32_t v) {
-  v = min(v, dpp_u32<kDppXor1>(v));
-  v = min(v, dpp_u32<kDppXor2>(v));
-  return min(v, dpp_u32<kDppHalfMirror>(v));
+constexpr int kDppShr1 = 0x111;          // lane i <- i - 1 within each row of 16
+constexpr int kDppBcast = 0x150;         // + n: lane n of each row to all of it
+// Lane 7 of the vector's 8 lanes to all of them (banks 0, 1 hold the row's
+// first vector, 2, 3 its second).
+__device__ __forceinline__ uint32_t last8(uint32_t v) {
+  const int lo = __builtin_amdgcn_update_dpp((int)v, (int)v, kDppBcast + 7, 0xF, 0x3, false);
+  return (uint32_t)__builtin_amdgcn_update_dpp(lo, (int)v, kDppBcast + 15, 0xF, 0xC, false);
 }
+// Over the 8 lanes of a vector.
 __device__ __forceinline__ uint32_t or8(uint32_t v) {
   v |= dpp_u32<kDppXor1>(v);
   v |= dpp_u32<kDppXor2>(v);
   return v | dpp_u32<kDppHalfMirror>(v);
 }
 
-// nv rows of d halves between memory and LDS rows of kVecRow halves; 16-byte
-// accesses where d is a multiple of 8 and the base 16-byte aligned.
-__device__ __forceinline__ void vec_rows_in(const uint16_t* src, uint16_t* rows, int nv, int d, bool wide, int lane) {
+// A vector's row of d halves between memory and LDS, by its own 8 lanes;
+// 16-byte accesses where d is a multiple of 8 and the base 16-byte aligned.
+__device__ __forceinline__ void vec_row_in(const uint16_t* src, uint16_t* row, int d, bool wide, int l8) {
   if (wide) {
-    const int per = d / 8;
-    for (int i = lane; i < nv * per; i += kWave)
-      *reinterpret_cast<u32x4*>(rows + i / per * kVecRow + i % per * 8) = load16(src + 8 * i);
+    for (int i = 8 * l8; i < d; i += 8 * kVecLanes) *reinterpret_cast<u32x4*>(row + i) = load16(src + i);
   } else {
-    for (int i = lane; i < nv * d; i += kWave) rows[i / d * kVecRow + i % d] = src[i];
+    for (int i = l8; i < d; i += kVecLanes) row[i] = src[i];
   }
 }
-__device__ __forceinline__ void vec_rows_out(uint16_t* dst, const uint16_t* rows, int nv, int d, bool wide, int lane) {
+__device__ __forceinline__ void vec_row_out(uint16_t* dst, const uint16_t* row, int d, bool wide, int l8) {
   if (wide) {
-    const int per = d / 8;
-    for (int i = lane; i < nv * per; i += kWave)
-      *reinterpret_cast<u32x4*>(dst + 8 * i) = *reinterpret_cast<const u32x4*>(rows + i / per * kVecRow + i % per * 8);
+    for (int i = 8 * l8; i < d; i += 8 * kVecLanes)
+      *reinterpret_cast<u32x4*>(dst + i) = *reinterpret_cast<const u32x4*>(row + i);
   } else {
-    for (int i = lane; i < nv * d; i += kWave) dst[i] = rows[i / d * kVecRow + i % d];
+    for (int i = l8; i < d; i += kVecLanes) dst[i] = row[i];
   }
+}
+// The same for a record's n bytes, in dwords where `dwords`.
+__device__ __forceinline__ void vec_bytes(uint8_t* dst, const uint8_t* src, int n, bool dwords, int l8) {
+  int done = 0;
+  if (dwords) {
+#pragma unroll 4
+    for (int i = 4 * l8; i + 4 <= n; i += 4 * kVecLanes)
+      *reinterpret_cast<uint32_t*>(dst + i) = *reinterpret_cast<const uint32_t*>(src + i);
+    done = n & ~3;
+  }
+  for (int i = done + l8; i < n; i += kVecLanes) dst[i] = src[i];
 }
 
 // Bytes of a record that are written (the stride can be longer: the last
@@ -107,39 +148,45 @@ __global__ __launch_bounds__(kWave) void kivi_vec_compress_kernel(
   uint16_t* x = s_x + vi * kVecRow;
   uint16_t* res = s_res + vi * kVecRow;
   uint8_t* rec = s_rec + vi * kVecRec;
-  vec_rows_in(in + v0 * head_dim, s_x, nv, head_dim, wide, lane);
+  if (vi < nv) vec_row_in(in + (v0 + vi) * head_dim, x, head_dim, wide, l8);
   // channels up to the next multiple of 8: NaN, which the scan skips
   if (vi < nv && head_dim + l8 < (head_dim + 7) / 8 * 8) x[head_dim + l8] = 0x7FFF;
   __syncthreads();
 
   // Top-n_outliers |x| by the reference's replace-the-first-minimum scan.  A
   // slot is one word: (|x| as ordered bits + 1, 0 when empty) << 16 | slot
-  // << 8 | channel, so the least word of the vector's slots is the first
-  // slot of least magnitude.
+  // << 8 | 255 - channel.  The words stand in descending order over places
+  // 8 i + l8 (the last n_outliers of them), so the first slot of least
+  // magnitude is the last place, and its slot goes to the channel that
+  // replaces it: that word enters at its place and those below it move on
+  // by one, all of which is the median of (own word, word before, new word).
+  // A channel no greater than the least falls below the last place: at equal
+  // magnitude its word has that slot and a smaller channel field.
   uint32_t key[SPL];
 #pragma unroll
   for (int i = 0; i < SPL; ++i) {
-    const int s = i * kVecLanes + l8;
-    key[i] = s < n_outliers ? (uint32_t)s << 8 : 0xFFFFFFFFu;
+    const int s = SPL * kVecLanes - 1 - (i * kVecLanes + l8);
+    key[i] = s < n_outliers ? (uint32_t)s << 8 | 0xFFu : 0xFFFFFFFFu;
   }
   if (n_outliers > 0) {
-    uint32_t least = 0;                               // slot 0, empty
+    const uint32_t top = l8 == 0 ? 0xFFFFFFFFu : 0u;
     for (int d0 = 0; d0 < head_dim; d0 += 8) {
       const u32x4 c = *reinterpret_cast<const u32x4*>(x + d0);
       const uint32_t w[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const uint32_t m = ((w[e / 2] >> (16 * (e & 1))) & 0x7FFFu) + 1u;
-        const bool take = m > (least >> 16) && m <= 0x7C01u;      // greater, and not NaN
-        const uint32_t put = m << 16 | (least & 0xFF00u) | (uint32_t)(d0 + e);
-        const uint32_t at = take ? least : 0xFFFFFFFEu;           // no slot holds that word
-        uint32_t lo = 0xFFFFFFFFu;
+        const uint32_t h = (w[e / 2] >> (16 * (e & 1))) & 0x7FFFu;
+        const uint32_t m = (h <= 0x7C00u ? (h + 1u) << 16 : 0u) | (uint32_t)(255 - d0 - e);   // NaN is never greater
+        uint32_t last[SPL], before[SPL];
 #pragma unroll
         for (int i = 0; i < SPL; ++i) {
-          key[i] = key[i] == at ? put : key[i];
-          lo = min(lo, key[i]);
+          last[i] = last8(key[i]);
+          before[i] = dpp_u32<kDppShr1>(key[i]) | top;
+          if (i > 0) before[i] = l8 == 0 ? last[i - 1] : before[i];
         }
-        least = min8(lo);
+        const uint32_t put = (last[SPL - 1] & 0xFF00u) | m;
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) key[i] = max(key[i], min(put, before[i]));
       }
     }
   }
@@ -149,9 +196,8 @@ __global__ __launch_bounds__(kWave) void kivi_vec_compress_kernel(
   uint32_t mask[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int i = 0; i < SPL; ++i) {
-    const int s = i * kVecLanes + l8;
-    if (s < n_outliers) {
-      const int ch = key[i] & 0xFF;
+    if (key[i] != 0xFFFFFFFFu) {
+      const int s = key[i] >> 8 & 0xFF, ch = 255 - (key[i] & 0xFF);
       const uint16_t h = x[ch];
       rec[3 * s] = (uint8_t)ch;
       rec[3 * s + 1] = (uint8_t)(h & 0xff);
@@ -173,11 +219,11 @@ __global__ __launch_bounds__(kWave) void kivi_vec_compress_kernel(
     if (l8 & 1) before += __builtin_popcount(mine & 0xFFFFu);
     const uint32_t own = (l8 & 1) ? mine >> 16 : mine;
     int r = 16 * l8 - before;
+    const u32x4 c[2] = {*reinterpret_cast<const u32x4*>(x + 16 * l8), *reinterpret_cast<const u32x4*>(x + 16 * l8 + 8)};
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int d = 16 * l8 + e;
-      const bool put = !((own >> e) & 1u) && d < head_dim;
-      if (put && r < n_res) res[r] = x[d];
+      const bool put = !((own >> e) & 1u) && 16 * l8 + e < head_dim;
+      if (put && r < n_res) res[r] = (uint16_t)(word(c[e / 8], e % 8 / 2) >> (16 * (e & 1)));
       r += put ? 1 : 0;
     }
   }
@@ -189,91 +235,103 @@ __global__ __launch_bounds__(kWave) void kivi_vec_compress_kernel(
     // groups start at even indices: pairs are whole words
     const uint32_t* pairs = reinterpret_cast<const uint32_t*>(res + g0);
     const int n = g1 - g0;
+    uint8_t* p = rec + 3 * n_outliers + g * (group_size / 2 + 4);
     float gmin = FLT_MAX, gmax = -FLT_MAX;
+    bool in_order = true;
+    if (n % 2 == 0) {
+      half2v a = as_half2(pairs[0]), b = a;
 #pragma unroll 4
-    for (int i = 0; i < n; i += 2) {
-      const uint32_t w = pairs[i / 2];
-      const float a = f16_to_f32((uint16_t)w), b = i + 1 < n ? f16_to_f32((uint16_t)(w >> 16)) : a;
-      if (a < gmin) gmin = a;
-      if (a > gmax) gmax = a;
-      if (b < gmin) gmin = b;
-      if (b > gmax) gmax = b;
+      for (int i = 1; i < n / 2; ++i) {
+        a = pk_min(a, as_half2(pairs[i]));
+        b = pk_max(b, as_half2(pairs[i]));
+      }
+      gmin = (float)__builtin_elementwise_minimum(a.x, a.y);
+      gmax = (float)__builtin_elementwise_maximum(b.x, b.y);
+      in_order = scan_in_order(gmin, gmax);
+    }
+    if (in_order) {
+      gmin = FLT_MAX;
+      gmax = -FLT_MAX;
+      for (int i = 0; i < n; ++i) {
+        const float a = f16_to_f32(res[g0 + i]);
+        if (a < gmin) gmin = a;
+        if (a > gmax) gmax = a;
+      }
     }
     const GroupQ q = group_params(gmin, gmax);
-    uint8_t* p = rec + 3 * n_outliers + g * (group_size / 2 + 4);
+    if (!in_order) {
 #pragma unroll 4
-    for (int i = 0; i < n; i += 2) {
-      const uint32_t w = pairs[i / 2];
-      const int q0 = quantise(f16_to_f32((uint16_t)w), q);
-      const int q1 = i + 1 < n ? quantise(f16_to_f32((uint16_t)(w >> 16)), q) : 0;
-      *p++ = (uint8_t)((q1 << 4) | q0);
+      for (int i = 0; i < n / 2; ++i) {
+        const half2v w = as_half2(pairs[i]);
+        p[i] = (uint8_t)(biased_code(w.x, 1.0f, q.gmin, q.scale) + (biased_code(w.y, 1.0f, q.gmin, q.scale) << 4));
+      }
+    } else {
+      for (int i = 0; i < n; i += 2) {
+        const int q0 = quantise(f16_to_f32(res[g0 + i]), q);
+        const int q1 = i + 1 < n ? quantise(f16_to_f32(res[g0 + i + 1]), q) : 0;
+        p[i / 2] = (uint8_t)((q1 << 4) | q0);
+      }
     }
+    p += (n + 1) / 2;
     p[0] = (uint8_t)(q.step & 0xff); p[1] = (uint8_t)(q.step >> 8);
     p[2] = (uint8_t)(q.zero & 0xff); p[3] = (uint8_t)(q.zero >> 8);
   }
   __syncthreads();
 
-  uint8_t* dst = out + v0 * stride;
-  const int words = rec_bytes / 4;
-  int done = 0;
-  if (dwords) {
-    for (int i = lane; i < nv * words; i += kWave) {
-      const int v = i / words, w = i % words;
-      *reinterpret_cast<uint32_t*>(dst + (int64_t)v * stride + 4 * w) =
-          *reinterpret_cast<const uint32_t*>(s_rec + v * kVecRec + 4 * w);
-    }
-    done = 4 * words;
-  }
-  const int rest = rec_bytes - done;
-  for (int i = lane; i < nv * rest; i += kWave) {
-    const int v = i / rest, b = done + i % rest;
-    dst[(int64_t)v * stride + b] = s_rec[v * kVecRec + b];
-  }
+  if (vi < nv) vec_bytes(out + (v0 + vi) * stride, rec, rec_bytes, dwords, l8);
 }
 
 __global__ __launch_bounds__(kWave) void kivi_vec_decompress_kernel(
     const uint8_t* __restrict__ in, uint16_t* __restrict__ out, int n_vecs, int head_dim, int n_outliers,
     int group_size, int stride, int rec_bytes, bool wide, bool dwords) {
   __shared__ __attribute__((aligned(16))) uint16_t s_x[kVecVecs * kVecRow];
+  __shared__ __attribute__((aligned(16))) uint16_t s_res[kVecVecs * kVecRow];
   __shared__ __attribute__((aligned(16))) uint8_t s_rec[kVecVecs * kVecRec];
   const int lane = threadIdx.x, l8 = lane % kVecLanes, vi = lane / kVecLanes;
   const int64_t v0 = (int64_t)blockIdx.x * kVecVecs;
   const int nv = (int)min<int64_t>(kVecVecs, n_vecs - v0);
-  const uint8_t* src = in + v0 * stride;
-  {
-    const int words = rec_bytes / 4;
-    int done = 0;
-    if (dwords) {
-      for (int i = lane; i < nv * words; i += kWave) {
-        const int v = i / words, w = i % words;
-        *reinterpret_cast<uint32_t*>(s_rec + v * kVecRec + 4 * w) =
-            *reinterpret_cast<const uint32_t*>(src + (int64_t)v * stride + 4 * w);
+  uint8_t* rec = s_rec + vi * kVecRec;
+  uint16_t* x = s_x + vi * kVecRow;
+  uint16_t* res = s_res + vi * kVecRow;
+  if (vi < nv) vec_bytes(rec, in + (v0 + vi) * stride, rec_bytes, dwords, l8);
+  __syncthreads();
+  const int n_res = head_dim - n_outliers;
+  if (vi < nv) {
+    // the groups' values, ascending, a group per lane
+    const int n_groups = (n_res + group_size - 1) / group_size;
+    for (int g = l8; g < n_groups; g += kVecLanes) {
+      const int n = min(group_size, n_res - g * group_size), nb = (n + 1) / 2;
+      const uint8_t* pack = rec + 3 * n_outliers + g * (group_size / 2 + 4);
+      const uint8_t* p = pack + nb;
+      const float st = f16_to_f32((uint16_t)(p[0] | (p[1] << 8)));
+      const float ze = f16_to_f32((uint16_t)(p[2] | (p[3] << 8)));
+      // groups start at even indices: pairs are whole words (the last pair's
+      // second value is not read when there is none)
+      uint32_t* pairs = reinterpret_cast<uint32_t*>(res + g * group_size);
+#pragma unroll 4
+      for (int i = 0; i < nb; ++i) {
+        const int b = pack[i];
+        pairs[i] = f32_to_f16(__builtin_fmaf((float)(b & 0x0f), st, ze)) |
+                   (uint32_t)f32_to_f16(__builtin_fmaf((float)(b >> 4), st, ze)) << 16;
       }
-      done = 4 * words;
-    }
-    const int rest = rec_bytes - done;
-    for (int i = lane; i < nv * rest; i += kWave) {
-      const int v = i / rest, b = done + i % rest;
-      s_rec[v * kVecRec + b] = src[(int64_t)v * stride + b];
     }
   }
   __syncthreads();
   if (vi < nv) {
-    const uint8_t* rec = s_rec + vi * kVecRec;
-    uint16_t* x = s_x + vi * kVecRow;
     // lane l8 owns channels 16 l8 .. + 15; every lane reads every outlier,
     // so that of two for one channel the later stands
     uint32_t own = 0;
+#pragma unroll 4
     for (int i = 0; i < n_outliers; ++i) {
       const int ch = rec[3 * i];
+      const uint16_t h = (uint16_t)(rec[3 * i + 1] | (rec[3 * i + 2] << 8));
       if (ch / 16 == l8 && ch < head_dim) {
         own |= 1u << (ch % 16);
-        x[ch] = f32_to_f16(f16_to_f32((uint16_t)(rec[3 * i + 1] | (rec[3 * i + 2] << 8))));
+        x[ch] = f32_to_f16(f16_to_f32(h));
       }
     }
     // the other channels' ranks: those of the lanes before first
-    const int c1 = min(16 * l8 + 16, head_dim);
-    const int owned = max(c1 - 16 * l8, 0);
+    const int owned = max(min(16 * l8 + 16, head_dim) - 16 * l8, 0);
     const int free_own = owned - __builtin_popcount(own);
     int before = 0;
 #pragma unroll
@@ -281,28 +339,16 @@ __global__ __launch_bounds__(kWave) void kivi_vec_decompress_kernel(
       const int n = __shfl(free_own, (lane & ~(kVecLanes - 1)) + ((l8 - o) & (kVecLanes - 1)), kWave);
       before += o <= l8 ? n : 0;
     }
-    const int n_res = head_dim - n_outliers;
-    const int last0 = (n_res - 1) / group_size * group_size;        // first index of the last group
-    int r = before;
-    for (int e = 0; e < owned; ++e) {
-      if ((own >> e) & 1u) continue;
-      float val = 0.f;
-      if (r < n_res) {
-        const int g = r / group_size, k = r - g * group_size;
-        const uint8_t* pack = rec + 3 * n_outliers + g * (group_size / 2 + 4);
-        const int n = g * group_size == last0 ? n_res - last0 : group_size;
-        const uint8_t* p = pack + (n + 1) / 2;
-        const float st = f16_to_f32((uint16_t)(p[0] | (p[1] << 8)));
-        const float ze = f16_to_f32((uint16_t)(p[2] | (p[3] << 8)));
-        const int nib = (k % 2 == 0) ? (pack[k / 2] & 0x0f) : (pack[k / 2] >> 4);
-        val = __builtin_fmaf((float)nib, st, ze);
-      }
-      x[16 * l8 + e] = f32_to_f16(val);
-      ++r;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      // channels past the values (two outliers for one channel) read as zero
+      const int r = before + e - __builtin_popcount(own & ((1u << e) - 1u));
+      const uint16_t v = r < n_res ? res[r] : (uint16_t)0;
+      if (e < owned && !((own >> e) & 1u)) x[16 * l8 + e] = v;
     }
   }
   __syncthreads();
-  vec_rows_out(out + v0 * head_dim, s_x, nv, head_dim, wide, lane);
+  if (vi < nv) vec_row_out(out + (v0 + vi) * head_dim, x, head_dim, wide, l8);
 }
 
 // ---------------------------------------------------------------------------
@@ -364,34 +410,6 @@ __global__ __launch_bounds__(128) void kivi_append_kernel(PageJob j) {
 // (79.9 before).  Held to fewer registers for 5 or 6 wavefronts per SIMD (116
 // here, 4) it spills: 46 and 54 us.
 // ---------------------------------------------------------------------------
-
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-// Least and greatest of packed halves, element by element; a NaN stays.
-__device__ __forceinline__ half2v pk_min(half2v a, half2v b) { return __builtin_elementwise_minimum(a, b); }
-__device__ __forceinline__ half2v pk_max(half2v a, half2v b) { return __builtin_elementwise_maximum(a, b); }
-__device__ __forceinline__ half2v as_half2(uint32_t w) { return __builtin_bit_cast(half2v, w); }
-
-// The scans of group_params' caller start from +-FLT_MAX, skip NaN and keep
-// the first of equal values.  Over finite values that is the plain least and
-// greatest value, but for the sign of a zero minimum: such groups, and those
-// with a NaN or an infinity, are scanned in order.
-__device__ __forceinline__ bool scan_in_order(float mn, float mx) {
-  return !(mn > -FLT_MAX && mx < FLT_MAX) || mn == 0.0f;
-}
-
-// The codes of quantise over a group of finite values, before packing: the
-// code plus kCodeBias.  x - min is exact in one rounding from the half, the
-// product is rounded by itself (no contraction), and it lies in [0, LEVELS]
-// up to a rounding, so adding 2^23 leaves its nearest-even integer in the low
-// mantissa bits and no clamp is needed.
-constexpr uint32_t kCodeBias = 0x4B000000u;                      // 2^23 in fp32
-__device__ __forceinline__ uint32_t biased_code(_Float16 x, float one, float gmin, float scale) {
-#pragma clang fp contract(off)
-  const float d = __builtin_fmaf((float)x, one, -gmin);
-  const float p = d * scale;
-  return __float_as_uint(p + 8388608.0f);
-}
 
 // N codes of BITS each (8 of 4 bits, 4 of 8) into a dword, code i at bit
 // shift_of(i).
