@@ -6,6 +6,7 @@
 #include "tl_internal.hpp"
 #include "tl_kivi.hpp"
 
+#include <algorithm>
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -862,6 +863,32 @@ static void kivi_plan(const tl_kivi_desc* d, int32_t max_ctx, bool rope, int* P,
     if (want < 1) want = 1;
     if (want > pages) want = pages;
     pp = (int)((pages + want - 1) / want);
+    // Grids of an eighth of the CUs' workgroups and more do better with fewer
+    // partitions than 512 workgroups need: each costs its start (page ids,
+    // rotations) and the merge.  Below 144 items about one workgroup per CU,
+    // the last partition with fewer pages, by what its fp16 window and the
+    // append take beside pages (45 at a window of 128, at most half the
+    // pages); up to 256 items a single pass, as from 448 on and, at 4 bits, in
+    // between.  Longer contexts keep 512 workgroups, as INT4 at 256 items does
+    // with keys held before RoPE, where the rotation of a page, and not the
+    // start, is what counts.
+    // us, the step at 2900 tokens, INT8 before RoPE / INT8 / INT4 before RoPE
+    // / INT4 (32/8 heads, window 128): 16 sequences 46.1, 35.4, 40.4, 27.2
+    // before and 41.2, 30.7, 35.3, 23.4 now; 24: 64, 51, 56, 35 and 59, 41,
+    // 51, 29; 56: 107, 91, 81, 56 and 92, 86, 66, 48.  Past the lines: 32
+    // INT4 before RoPE 47.9 split, 51.2 single; 48 INT8 74 and 80; 20 of 8000
+    // tokens, INT8, 83 and 92.
+    const bool int4 = kivi_bits(d) == 4;
+    if (items >= 64 && items < 144) {
+      const long parts = (256 + items / 2) / items;
+      const long window = std::min<long>(10L * (d->residual_length + 16) / 32, pages / 2);
+      const long even = (pages + window + parts - 1) / parts;
+      if (even <= (int4 || rope ? 100 : 90)) pp = (int)std::min((long)pages, even);
+    } else if ((items >= 144 && items <= 256 && pages <= 192 && !(items == 256 && int4 && rope)) ||
+               (items >= 448 && items < 512 && pages <= 100) ||
+               (items > 256 && items < 448 && int4 && pages <= 100)) {
+      pp = pages;
+    }
   }
   if (pp > tl::kKiviMaxWgPages) pp = tl::kKiviMaxWgPages;   // a workgroup stages its page ids in LDS
   if (rope && pp > tl::kivi_page_rot_cap(kivi_bits(d))) pp = tl::kivi_page_rot_cap(kivi_bits(d));
