@@ -33,9 +33,9 @@
 // a workgroup barrier after every phase, so that on each SIMD one
 // wavefront's matrix ops run beside the other's VALU work.
 // Decode rows run the matrix-core decode wavefronts (tl_mfma_wave.hpp), one
-// workgroup per (sequence, kv head, 16-head slice), as a second kernel of the
-// same call on the same stream (one kernel for both would be sized by the
-// decode path's registers on top of the prefill path's).
+// workgroup per (sequence, kv head, 16-head slice): after the tiles in their
+// launch where the rows are few (rows_with_tiles), else as a kernel of their
+// own before it on the same stream.
 // Pools: f16 / bf16 (the q type), or FP8 E4M3 with per-tensor k_scale /
 // v_scale (codes converted exactly to the q type for q.k and to f16 for
 // p.v as they are staged; k_scale folds into the score scale, v_scale into
@@ -130,8 +130,15 @@ struct PrefillParams {
   int pf_seqs;                 // sequences [0, pf_seqs) may be prefill rows
   int dec_first;               // sequences [dec_first, num_seqs) may be decode rows
   int split;                   // prefill tiles: prefill_split_kernel
+  int pf_wgs;                  // prefill_kernel: workgroups of its tiles (those of decode rows follow)
 };
 
+// LDS of a decode row's workgroup.
+template <int NW>
+struct DecodeRowSmem {
+  float acc[NW * mw::kHeads * kPfHead];
+  float m[NW * mw::kHeads], l[NW * mw::kHeads];
+};
 template <int NW>
 struct PrefillSmem {
   struct {
@@ -193,8 +200,31 @@ __device__ __forceinline__ u32x4 fp8x8_to(const u32x4& c) {
   return u32x4{cvt(c.x, false), cvt(c.x, true), cvt(c.y, false), cvt(c.y, true)};
 }
 
-// Q: the q / out type (f16 or bf16); KV: the pool's, Q or FP8.
+// Decode rows (q_len == 1) of a mixed batch, one workgroup per (sequence,
+// kv head, 16-head slice), q / out row cu_q_lens[s]: the matrix-core decode
+// wavefronts (tl_mfma_wave.hpp), so a GQA group of up to 16 heads reads its
+// KV once, at every block size and for FP8 pools too.
 template <Kind Q, Kind KV, int BS, int NW>
+__device__ __forceinline__ void decode_row(const PrefillParams& pp, int b, DecodeRowSmem<NW>& sm) {
+  constexpr int GT = mw::kHeads;
+  const Params& p = pp.base;
+  const int slices = (p.group + GT - 1) / GT;
+  const int hs = b % slices; b /= slices;
+  const int kvh = b % p.num_kv_heads, seq = pp.dec_first + b / p.num_kv_heads;
+  const int q0 = pp.cu_q_lens[seq];
+  if (pp.cu_q_lens[seq + 1] - q0 != 1) return;
+  const int L = p.seq_lens[seq];
+  Params pd = p;
+  const int64_t shift = (int64_t)(q0 - seq) * p.num_heads * kPfHead * 2;   // q / out row q0
+  pd.q = (const char*)p.q + shift;
+  pd.out = (char*)p.out + shift;
+  pd.head_slices = slices;
+  mw::decode_workgroup<KV, Q, Kind::F32, NW, true, BS>(pd, seq, kvh, hs, 0, 0, L, sm.acc, sm.m, sm.l);
+}
+
+// Q: the q / out type (f16 or bf16); KV: the pool's, Q or FP8.  ROWS: decode
+// rows follow the tiles in the launch (rows_with_tiles).
+template <Kind Q, Kind KV, int BS, int NW, bool ROWS>
 __global__ __launch_bounds__(NW * kWave) void prefill_kernel(PrefillParams pp) {
   static_assert(BS >= 8 && BS <= 256 && (BS & (BS - 1)) == 0, "block size: a power of two 8 .. 256");
   static_assert(NW == 8, "two groups of four wavefronts, one wavefront of each group per SIMD");
@@ -205,7 +235,16 @@ __global__ __launch_bounds__(NW * kWave) void prefill_kernel(PrefillParams pp) {
   constexpr int E = KV == Kind::FP8 ? 1 : 2;              // pool bytes per element
   using M = Mfma32<Q>;                                 // q.k
   using MP = Mfma32<Kind::F16>;                        // p.v (f16 for every type)
-  __shared__ __attribute__((aligned(16))) PrefillSmem<NW> sm;
+  union Smem { PrefillSmem<NW> pf; DecodeRowSmem<ROWS ? NW : 1> dec; };
+  __shared__ __attribute__((aligned(16))) Smem smem;
+  auto& sm = smem.pf;
+  const int b0 = blockIdx.x;
+  if constexpr (ROWS) {
+    if (b0 >= pp.pf_wgs) {
+      decode_row<Q, KV, BS, NW>(pp, b0 - pp.pf_wgs, smem.dec);
+      return;
+    }
+  }
 
   const Params& p = pp.base;
   const int tid = threadIdx.x, lane = tid % kWave;
@@ -215,10 +254,9 @@ __global__ __launch_bounds__(NW * kWave) void prefill_kernel(PrefillParams pp) {
   // wavefront w runs on SIMD w % 4, so every SIMD holds one of each
   const int grp = wave >> 2;
 
-  int b = blockIdx.x;
   const int items = pp.pf_seqs * p.num_kv_heads;
-  const int tile = pp.row_tiles - 1 - b / items;       // longest (latest) tiles first
-  b %= items;
+  const int tile = pp.row_tiles - 1 - b0 / items;      // longest (latest) tiles first
+  const int b = b0 % items;
   const int seq = b / p.num_kv_heads, kvh = b % p.num_kv_heads;
   // The table entries of the wavefront's key group (see the staging below)
   // in the first two iterations are read with the lengths, before the exits
@@ -787,7 +825,7 @@ struct PrefillSplitSmem {
   float m[kSplitNW][kPfRows], l[kSplitNW][kPfRows];
 };
 
-template <Kind Q, Kind KV, int BS>
+template <Kind Q, Kind KV, int BS, bool ROWS>
 __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(PrefillParams pp) {
   static_assert(BS >= 8 && BS <= 256 && (BS & (BS - 1)) == 0, "block size: a power of two 8 .. 256");
   static_assert(KV == Q || KV == Kind::FP8, "a 2-byte pool holds the q type");
@@ -797,7 +835,16 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   constexpr int E = KV == Kind::FP8 ? 1 : 2;              // pool bytes per element
   using M = Mfma32<Q>;                                 // q.k
   using MP = Mfma32<Kind::F16>;                        // p.v (f16 for every type)
-  __shared__ __attribute__((aligned(16))) PrefillSplitSmem sm;
+  union Smem { PrefillSplitSmem pf; DecodeRowSmem<ROWS ? kSplitNW : 1> dec; };
+  __shared__ __attribute__((aligned(16))) Smem smem;
+  auto& sm = smem.pf;
+  const int b0 = blockIdx.x;
+  if constexpr (ROWS) {
+    if (b0 >= pp.pf_wgs) {
+      decode_row<Q, KV, BS, kSplitNW>(pp, b0 - pp.pf_wgs, smem.dec);
+      return;
+    }
+  }
 
   const Params& p = pp.base;
   const int lane = threadIdx.x % kWave;
@@ -805,10 +852,9 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   const int g = lane >> 5, c32 = lane & 31;
   const int grp = wave / kSplitWaves, wr = wave % kSplitWaves;
 
-  int b = blockIdx.x;
   const int items = pp.pf_seqs * p.num_kv_heads;
-  const int tile = pp.row_tiles - 1 - b / items;       // longest (latest) tiles first
-  b %= items;
+  const int tile = pp.row_tiles - 1 - b0 / items;      // longest (latest) tiles first
+  const int b = b0 % items;
   const int seq = b / p.num_kv_heads, kvh = b % p.num_kv_heads;
   const int32_t* table = p.block_tables + (int64_t)seq * p.max_blocks_per_seq;
   // entries of iteration it: lane i (< BPI) holds that of block i
@@ -1148,29 +1194,28 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   }
 }
 
-// Decode rows (q_len == 1) of a mixed batch, one workgroup per (sequence,
-// kv head, 16-head slice), q / out row cu_q_lens[s]: the matrix-core decode
-// wavefronts (tl_mfma_wave.hpp), so a GQA group of up to 16 heads reads its
-// KV once, at every block size and for FP8 pools too.
+// The decode rows alone: calls without prefill tiles, or with few of them.
 template <Kind Q, Kind KV, int BS, int NW>
 __global__ __launch_bounds__(NW * kWave) void prefill_decode_kernel(PrefillParams pp) {
-  constexpr int GT = mw::kHeads;
-  __shared__ __attribute__((aligned(16))) float s_acc[NW * GT * kPfHead];
-  __shared__ float s_m[NW * GT], s_l[NW * GT];
-  const Params& p = pp.base;
-  const int slices = (p.group + GT - 1) / GT;
-  int b = blockIdx.x;
-  const int hs = b % slices; b /= slices;
-  const int kvh = b % p.num_kv_heads, seq = pp.dec_first + b / p.num_kv_heads;
-  const int q0 = pp.cu_q_lens[seq];
-  if (pp.cu_q_lens[seq + 1] - q0 != 1) return;
-  const int L = p.seq_lens[seq];
-  Params pd = p;
-  const int64_t shift = (int64_t)(q0 - seq) * p.num_heads * kPfHead * 2;   // q / out row q0
-  pd.q = (const char*)p.q + shift;
-  pd.out = (char*)p.out + shift;
-  pd.head_slices = slices;
-  mw::decode_workgroup<KV, Q, Kind::F32, NW, true, BS>(pd, seq, kvh, hs, 0, 0, L, s_acc, s_m, s_l);
+  __shared__ __attribute__((aligned(16))) DecodeRowSmem<NW> sm;
+  decode_row<Q, KV, BS, NW>(pp, blockIdx.x, sm);
+}
+
+// Whether a call's decode rows go with its tiles, after them, instead of in a
+// launch of their own before: a row's workgroup is a chain of round trips over
+// its keys, which few rows leave the GPU to wait for, while the tiles'
+// wavefronts (and the CUs past their last) could work.  Rows that fill the
+// GPU stream faster by themselves, and tiles in full rounds leave no CU.
+// Same context for prompts and rows, bf16, 32/8 heads, us, rows before the
+// tiles and with them: 1 prompt of 128 of 4000 keys, 17 rows 113 and 62.5, 3
+// rows 104 and 59.8, 500 of 1500, 3 rows 49.8 and 45.0, 17 rows 52 either way
+// (all of the split kernel); 1 of 2048 of 2048, 8 rows 98.8 and 74.1; 5 of
+// 333 of 333, 3 rows 29.9 and 20.9; 3 of 700 of 3000, 3 rows 138 and 120.
+// Past the line: 8 of 256 of 4000, 17 rows 200 and 205; 2 of 1024 of 1024, 64
+// rows, 64 heads 100 and 109; 8 of 512 of 2048 (1024 tiles), 3 rows, 64 heads
+// 313 and 321.
+inline bool rows_with_tiles(const PrefillParams& pp, unsigned tiles, unsigned rows) {
+  return rows > 0 && tiles > 0 && (pp.split ? tiles + rows <= 256 || rows <= 64 : tiles <= 512 && rows <= 64);
 }
 
 template <Kind Q, Kind KV, int BS>
@@ -1181,12 +1226,18 @@ int launch_prefill_t(const PrefillParams& pp, unsigned grid, hipStream_t stream)
   const Params& p = pp.base;
   constexpr int GT = mw::kHeads;
   const unsigned dgrid = (unsigned)((pp.num_seqs - pp.dec_first) * p.num_kv_heads * ((p.group + GT - 1) / GT));
-  if (dgrid > 0)
+  const bool rows = rows_with_tiles(pp, grid, dgrid);
+  if (dgrid > 0 && !rows)
     hipLaunchKernelGGL((prefill_decode_kernel<Q, KV, BS, NWD>), dim3(dgrid), dim3(NWD * kWave), 0, stream, pp);
-  if (grid > 0 && pp.split)
-    hipLaunchKernelGGL((prefill_split_kernel<Q, KV, BS>), dim3(grid), dim3(kSplitNW * kWave), 0, stream, pp);
-  else if (grid > 0)
-    hipLaunchKernelGGL((prefill_kernel<Q, KV, BS, NW>), dim3(grid), dim3(NW * kWave), 0, stream, pp);
+  if (grid > 0) {
+    auto go = [&](auto kernel, int waves) {
+      hipLaunchKernelGGL(kernel, dim3(grid + (rows ? dgrid : 0)), dim3(waves * kWave), 0, stream, pp);
+    };
+    if (pp.split && rows) go(prefill_split_kernel<Q, KV, BS, true>, kSplitNW);
+    else if (pp.split) go(prefill_split_kernel<Q, KV, BS, false>, kSplitNW);
+    else if (rows) go(prefill_kernel<Q, KV, BS, NW, true>, NW);
+    else go(prefill_kernel<Q, KV, BS, NW, false>, NW);
+  }
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
 
@@ -1247,6 +1298,7 @@ int launch_prefill(const PrefillLaunch& a) {
              (int64_t)a.max_blocks_per_seq * a.block_size > kPfKeys;
   if (pp.split && pp.row_tiles) pp.row_tiles = (a.max_q_len * p.group + kSplitRows - 1) / kSplitRows;
   const unsigned grid = (unsigned)(pp.row_tiles * pp.pf_seqs * a.num_kv_heads);
+  pp.pf_wgs = (int)grid;
   const bool bf16 = a.dtype == (int)Kind::BF16;
   if (fp8)
     return bf16 ? launch_prefill_bs<Kind::BF16, Kind::FP8>(pp, a.block_size, grid, a.stream)
