@@ -470,9 +470,8 @@ int tl_kivi_append(const tl_kivi_desc* desc, const void* key, const void* value,
                    void* stream);
 
 /* Split-K partials of the decode and the step: 0 when the plan runs a
- * single pass.  Sized for the _pre_rope entry points' plan (as many
- * partitions as the other one, or more past 160 / 144 pages), so one size
- * serves every entry point. */
+ * single pass.  Sized for the larger of the plans of the _pre_rope and the
+ * other entry points, so one size serves every entry point. */
 size_t tl_kivi_workspace_bytes(const tl_kivi_desc* desc, int32_t max_context_len);
 
 /* Decode attention over pages (tokens < Lq) and the fp16 pool (tokens >= Lq).

@@ -4,6 +4,7 @@ HIP call is made."""
 import ctypes
 
 import pytest
+import torch
 
 import tl_attn as tla
 
@@ -531,6 +532,43 @@ def test_kivi_rope_step_workspace_and_argument_checks():
     assert call(d, pos=None) == tla.ERR_INVALID_ARGUMENT
     assert call(_kdesc(head_size=64)) == tla.ERR_NOT_IMPLEMENTED
     assert call(_kdesc(num_seqs=0), ws=None, ws_bytes=0) == tla.OK
+
+
+# A call that passes every check launches: on the pointers above only where
+# there is no GPU (the launch then fails, with TL_ERR_BACKEND).
+no_gpu = pytest.mark.skipif(torch.cuda.is_available(), reason="accepted calls would launch on pointers to nothing")
+MISALIGNED = ctypes.c_void_p(0x1008)    # refused after the size of the workspace is found to be enough
+
+
+def _too_small(rc):
+    return rc == tla.ERR_INVALID_ARGUMENT and "needed" in tla.last_error()
+
+
+def _kivi_refused(d, ctx, given, rope):
+    """Whether the decode or the step refuses a workspace of `given` bytes as too small."""
+    L, p, ws = tla.lib, ctypes.byref(d), (MISALIGNED, given, None)
+    if rope:
+        tables = (FAKE, FAKE, 1 << 20, 0)
+        return (_too_small(L.tl_kivi_paged_attention_decode_pre_rope(p, *[FAKE] * 8, ctx, *tables, *ws)) or
+                _too_small(L.tl_kivi_decode_step_pre_rope(p, *[FAKE] * 11, ctx, *tables, *ws)))
+    return (_too_small(L.tl_kivi_paged_attention_decode(p, *[FAKE] * 8, ctx, *ws)) or
+            _too_small(L.tl_kivi_decode_step(p, *[FAKE] * 11, ctx, *ws)))
+
+
+@no_gpu
+@pytest.mark.parametrize("H,n_kv", [(32, 8), (64, 8), (32, 32), (8, 1)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_kivi_workspace_size_is_accepted_by_every_entry_point(bits, H, n_kv):
+    """The queried size against what the calls demand, over batches on both sides of every line of the plan and
+    contexts of 0 to 400 pages."""
+    for S in [1, 2, 3, 5, 7, 8, 9, 10, 12, 13, 15, 16, 17, 18, 20, 24, 27, 28, 31, 32, 33, 40, 47, 55, 56, 63, 64, 70]:
+        for ctx in [1, 140] + list(range(159, 13000, 32 * 7)) + [4480, 4600, 4800, 5090, 7400, 8160]:
+            for R in (128, 40):
+                for rope in (0, 1):
+                    d = _kdesc(num_seqs=S, num_heads=H, num_kv_heads=n_kv, bits=bits, residual_length=R,
+                               pre_rope_keys=rope)
+                    given = tla.kivi_workspace_bytes(d, ctx)
+                    assert not _kivi_refused(d, ctx, given, rope), (S, ctx, R, rope, tla.last_error())
 
 
 # ---- reference-named C++ operators (include/tl_truellm_ops.h) -------------

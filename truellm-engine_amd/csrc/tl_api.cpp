@@ -898,10 +898,14 @@ static void kivi_plan(const tl_kivi_desc* d, int32_t max_ctx, bool rope, int* P,
 
 size_t tl_kivi_workspace_bytes(const tl_kivi_desc* desc, int32_t max_context_len) {
   if (check_kivi(desc) != TL_OK || max_context_len < 0) return 0;
-  // the plan of the _pre_rope entry points: at least as many partitions as
-  // the other one, so the size serves both
-  int P, PP;
-  kivi_plan(desc, max_context_len, true, &P, &PP);
+  // the larger of the two plans, so that the size serves every entry point:
+  // either may run more partitions (the _pre_rope one past its pages per
+  // workgroup, the other where it alone keeps the split towards 512
+  // workgroups)
+  int P, P_rope, PP;
+  kivi_plan(desc, max_context_len, false, &P, &PP);
+  kivi_plan(desc, max_context_len, true, &P_rope, &PP);
+  P = std::max(P, P_rope);
   if (P <= 1) return 0;
   const size_t sh = (size_t)desc->num_seqs * desc->num_heads * P;
   return sh * desc->head_size * 4 + 2 * sh * 4;
