@@ -115,6 +115,22 @@ def test_auto_partitioning_targets_many_workgroups():
     assert tla.workspace_bytes(_desc(num_seqs=1, head_size=80), 4096) == 32 * 8 * (80 * 4 + 8)
 
 
+@pytest.mark.parametrize("kw", [dict(), dict(kv_dtype=tla.FP8_E4M3), dict(num_heads=64), dict(num_kv_heads=32),
+                                dict(head_size=80)])
+def test_workspace_of_a_longer_maximum_holds_for_shorter_contexts(kw):
+    """A program that sizes the workspace once, for its longest context, and passes each step's own maximum."""
+    for S in range(1, 80):
+        d = _desc(num_seqs=S, **kw)
+        sizes = [tla.workspace_bytes(d, 1 << k) for k in range(9, 18)]
+        assert sizes == sorted(sizes), (S, sizes)
+    d = _desc(num_seqs=16)
+    assert tla.workspace_bytes(d, 12000) <= tla.workspace_bytes(d, 20000)
+    for S, M in ((24, 20000), (32, 20000), (32, 16400), (40, 32768), (48, 20000)):
+        d = _desc(num_seqs=S, **kw)
+        most = tla.workspace_bytes(d, M)
+        assert all(tla.workspace_bytes(d, c) <= most for c in range(4608, M, 512)), (S, M)
+
+
 def test_v2_plan_inside_the_callers_scratch():
     """tl_paged_attention_v2's plan: f16 at head 128 keeps f16 partials, one
     partition per reference-kernel slot ((max_ctx / bs + 31) / 32); bf16 and

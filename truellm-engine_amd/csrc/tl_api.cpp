@@ -128,16 +128,11 @@ void plan_partitions(const tl_decode_desc* d, int32_t max_ctx, int* P, int* PT) 
     if (want > chunks) want = chunks;
     pt_chunks = (int)((chunks + want - 1) / want);
     if (want == 1 && chunks > 8) pt_chunks = 4;
-    if (uses_mfma(d)) {
-      // A grid that gives every CU one workgroup, or nearly two, runs single
-      // pass although it is below 512: splitting it evens nothing out and
-      // adds the merge.  2-byte KV otherwise runs at most 2048 tokens a
-      // partition up to 16384 tokens, as the full grids do.
-      const bool round = (items >= 224 && items <= 256 && chunks <= 16) || (items >= 448 && chunks <= 8);
-      const bool fp8 = d->kv_dtype == TL_DTYPE_FP8_E4M3;
-      if (round) pt_chunks = chunks;
-      else if (!fp8 && chunks > 8 && chunks <= 32 && pt_chunks > 4) pt_chunks = 4;
-    }
+    // A grid that gives every CU one workgroup, or nearly two, runs single
+    // pass although it is below 512: splitting it evens nothing out and adds
+    // the merge.
+    if (uses_mfma(d) && ((items >= 224 && items <= 256 && chunks <= 16) || (items >= 448 && chunks <= 8)))
+      pt_chunks = chunks;
   }
   if (pt_chunks < 1) pt_chunks = 1;
   *P = (chunks + pt_chunks - 1) / pt_chunks;
