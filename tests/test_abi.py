@@ -115,6 +115,19 @@ def test_auto_partitioning_targets_many_workgroups():
     assert tla.workspace_bytes(_desc(num_seqs=1, head_size=80), 4096) == 32 * 8 * (80 * 4 + 8)
 
 
+@pytest.mark.parametrize("kw,longest", [(dict(), 2048), (dict(num_heads=64), 2048), (dict(kv_dtype=tla.FP8_E4M3), 4096)])
+def test_grids_near_a_workgroup_per_cu_run_single_pass_over_short_contexts(kw, longest):
+    """224 .. 256 items and 448 and more, while an item's K and V are at most 1 MB; split past that, and split on
+    the other sides of the lines.  512 items: up to 4096 tokens, as ever."""
+    single = lambda S, ctx: tla.workspace_bytes(_desc(num_seqs=S, **kw), ctx) == 0
+    for S in (28, 30, 32, 56, 63):
+        assert single(S, 600) and single(S, longest)
+        assert not single(S, longest + 1) and not single(S, 8192)
+    for S in (27, 33, 55):
+        assert not single(S, 600) and not single(S, longest)
+    assert single(64, 4096) and not single(64, 4097)
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(kv_dtype=tla.FP8_E4M3), dict(num_heads=64), dict(num_kv_heads=32),
                                 dict(head_size=80)])
 def test_workspace_of_a_longer_maximum_holds_for_shorter_contexts(kw):

@@ -97,6 +97,18 @@ def test_bf16_llama_shape_variable_lengths(runner):
                  ATOL, runner)
 
 
+@pytest.mark.parametrize("longest", [2048, 2049])
+@pytest.mark.parametrize("S,code", [(28, orc.F16), (32, orc.BF16)])
+def test_uneven_batches_about_a_workgroup_per_cu(S, code, longest):
+    """224 and 256 (sequence, kv head) items, lengths from a sixteenth of the longest: single pass up to 2048
+    tokens, split past that."""
+    lens = inputs.uniform_lens(inputs.SEEDS[2] + S, S, longest // 16, longest)
+    lens[S // 2] = longest
+    case = inputs.make_paged_case(inputs.SEEDS[2], S, 32, 8, 128, 16, lens, code)
+    print(f"case uneven S={S} longest={longest}", flush=True)
+    assert_close(run_decode(case, tla.GQA_GROUPED), _ref(case, tla.GQA_GROUPED), code, ATOL, "auto")
+
+
 EDGE_LENS = [0, 1, 15, 16, 17, 511, 512, 513, 1023, 1025, 2047]
 
 

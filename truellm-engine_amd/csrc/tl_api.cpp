@@ -105,7 +105,8 @@ int check_decode(const tl_decode_desc* d) {
 // tokens and in 2048-token partitions past that: with lengths that differ
 // the single pass waits for its longest sequences (batch 64, lengths
 // uniform in [512, 8192], bf16: 172 us in 2048-token partitions against
-// 200 us single pass; equal lengths of 4096 would lose 3.5 %).
+// 200 us single pass; equal lengths of 4096 would lose 3.5 %).  Short
+// contexts of some smaller grids run single pass too (below).
 void plan_partitions(const tl_decode_desc* d, int32_t max_ctx, int* P, int* PT) {
   const int chunks = max_ctx > 0 ? (max_ctx + tl::kDecodeChunk - 1) / tl::kDecodeChunk : 1;
   if (d->partition_tokens > 0) {
@@ -129,9 +130,18 @@ void plan_partitions(const tl_decode_desc* d, int32_t max_ctx, int* P, int* PT) 
     pt_chunks = (int)((chunks + want - 1) / want);
     if (want == 1 && chunks > 8) pt_chunks = 4;
     // A grid that gives every CU one workgroup, or nearly two, runs single
-    // pass although it is below 512: splitting it evens nothing out and adds
-    // the merge.
-    if (uses_mfma(d) && ((items >= 224 && items <= 256 && chunks <= 16) || (items >= 448 && chunks <= 8)))
+    // pass although it is below 512, while the longest item holds at most 1 MB
+    // of K and V (2048 tokens of 2-byte KV, 4096 of FP8): the merge is then a
+    // larger part than what splitting evens out.  Split / single pass, equal
+    // lengths and the mean of five draws of uneven ones (from a sixteenth of
+    // the longest), 32/8 heads: bf16, 28 sequences of 1700 1.17 and 1.13, of
+    // 2048 1.14 and 1.12; 60 of 1300 1.13 and 1.07, of 2048 1.10 and 1.02; FP8,
+    // 28 of 4096 1.20 and 1.01, 60 of 4096 1.07 and 1.02.  Past the line, where
+    // uneven lengths lose: bf16, 28 of 3072 1.15 and 0.94, of 6000 1.06 and
+    // 0.95, of 8192 1.06 and 0.92; 60 of 3072 1.04 and 0.95; FP8, 28 of 8192
+    // 1.11 and 0.95.
+    const int single = d->kv_dtype == TL_DTYPE_FP8_E4M3 ? 8 : 4;   // chunks
+    if (uses_mfma(d) && ((items >= 224 && items <= 256) || items >= 448) && chunks <= single)
       pt_chunks = chunks;
   }
   if (pt_chunks < 1) pt_chunks = 1;
