@@ -600,6 +600,69 @@ def test_kivi_workspace_size_is_accepted_by_every_entry_point(bits, H, n_kv):
                     assert not _kivi_refused(d, ctx, given, rope), (S, ctx, R, rope, tla.last_error())
 
 
+def _kivi_even_partitions(d, ctx, rope):
+    """The split in equal page counts towards 512 workgroups."""
+    pages = tla.kivi_quantized_len(ctx, d.residual_length) // 32
+    if pages == 0:
+        return 1
+    items = d.num_seqs * d.num_kv_heads * -(-d.num_heads // d.num_kv_heads // 4)
+    per = -(-pages // min(pages, max(1, -(-512 // items))))
+    if rope:
+        per = min(per, 144 if d.bits == 8 else 160)
+    return -(-pages // per)
+
+
+@no_gpu
+@pytest.mark.parametrize("H,n_kv", [(32, 8), (64, 8), (8, 1)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_kivi_workspace_of_a_longer_maximum_holds_for_shorter_contexts(bits, H, n_kv):
+    """No plan asks for more than the even split's workspace, and no size that is not 0 is below it, so a workspace
+    sized once for the longest context holds wherever that of the even split would; a context whose plan is a
+    single pass has only such below it."""
+    for S in list(range(1, 40)) + [44, 50, 55, 56, 60, 63, 64]:
+        for R in (128, 40):
+            d = _kdesc(num_seqs=S, num_heads=H, num_kv_heads=n_kv, bits=bits, residual_length=R)
+            split = False
+            for pages in list(range(0, 24)) + list(range(24, 330, 11)) + [48, 49, 80, 81, 96, 100, 101]:
+                ctx = R + 32 * pages + 31
+                size = tla.kivi_workspace_bytes(d, ctx)
+                even = [S * H * _kivi_even_partitions(d, ctx, rope) * (128 * 4 + 8) for rope in (0, 1)]
+                assert size == 0 or size >= even[1], (S, R, pages)
+                for rope in (0, 1):
+                    d.pre_rope_keys = rope
+                    assert not _kivi_refused(d, ctx, even[rope], rope), (S, R, pages, rope, tla.last_error())
+                d.pre_rope_keys = 0
+            sizes = [tla.kivi_workspace_bytes(d, c) for c in range(R + 31, 9000, 32)]
+            first = next((i for i, n in enumerate(sizes) if n), len(sizes))
+            assert all(sizes[first:]), (S, R)
+
+
+@no_gpu
+def test_kivi_plan_lines():
+    """Single pass on one side of a line, split on the other (the plan's own partitions, from what the calls ask
+    for)."""
+    def parts(S, pages, bits, rope):
+        d = _kdesc(num_seqs=S, bits=bits, pre_rope_keys=rope)
+        per = S * 32 * (128 * 4 + 8)
+        return next(P for P in range(1, 65) if not _kivi_refused(d, 128 + 32 * pages, P * per if P > 1 else 0, rope))
+    for bits, rope in ((8, 1), (8, 0), (4, 1), (4, 0)):
+        for S in (17, 24, 27, 33, 40, 55):
+            assert parts(S, 24, bits, rope) == 1
+            assert (parts(S, 48, bits, rope) == 1) == (S < 33 or bits == 4 or rope == 1)
+        for S in (17, 24, 27):
+            assert parts(S, 49, bits, rope) > 1 and parts(S, 150, bits, rope) > 1
+        for S in (33, 55):
+            assert (parts(S, 49, bits, rope) == 1) == (parts(S, 80, bits, rope) == 1) == (bits == 4)
+        for S in (28, 30, 31, 32):
+            assert parts(S, 80, bits, rope) == 1 and parts(S, 81, bits, rope) > 1
+        for S in (56, 63):
+            assert parts(S, 100, bits, rope) == 1 and parts(S, 101, bits, rope) > 1
+    # one workgroup per CU: partitions with the window's shorter by 45 pages, else the even split
+    assert [parts(16, 86, bits, rope) for bits, rope in ((8, 1), (8, 0), (4, 1), (4, 0))] == [2, 2, 2, 2]
+    assert [parts(16, 124, bits, rope) for bits, rope in ((8, 1), (8, 0), (4, 1), (4, 0))] == [4, 2, 4, 2]
+    assert [parts(10, 86, bits, rope) for bits, rope in ((8, 1), (8, 0), (4, 1), (4, 0))] == [2, 7, 2, 2]
+
+
 # ---- reference-named C++ operators (include/tl_truellm_ops.h) -------------
 
 def _demangled_exports():

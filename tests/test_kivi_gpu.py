@@ -322,6 +322,36 @@ def test_kivi_decode_matches_oracle(pp, bits):
     assert_close(_run_decode(kc, pages, pp), _kivi_ref(kc, pages), orc.F16, ATOL_KIVI, f"pp={pp} bits={bits}")
 
 
+@pytest.mark.parametrize("S,pages", [(9, 40), (14, 60), (18, 48), (18, 49)])
+@pytest.mark.parametrize("bits,rope", [(4, 0), (8, 1)])
+def test_kivi_uneven_batches_with_the_library_plan(bits, rope, S, pages):
+    """Lengths from a sixteenth of the longest: partitions of unequal page counts (72 and 112 items: the window's
+    has fewer), a single pass of 144 items and the split past its line."""
+    longest = 128 + 32 * pages + 5
+    lens = inputs.uniform_lens(inputs.SEEDS[3] + S, S, longest // 16, longest)
+    lens[S // 2] = longest
+    kc = KiviCase(68, lens, bits=bits, extra_blocks=0)
+    pages_np = kc.oracle_pages()
+    print(f"case kivi uneven S={S} pages={pages} bits={bits} rope={rope}", flush=True)
+    if not rope:
+        assert_close(_run_decode(kc, pages_np), _kivi_ref(kc, pages_np), orc.F16, ATOL_KIVI, "uneven")
+        return
+    from test_oracle import rope_tables
+    cos_t, sin_t = rope_tables(longest, 128)
+    qd, kd, vd = dev(kc.q, orc.F16), dev(kc.k, orc.F16), dev(kc.v, orc.F16)
+    btd, sld, ptd = dev(kc.tables), dev(kc.lens), dev(kc.page_tables)
+    desc = kc.desc(qd, kd, btd, ptd)
+    desc.pre_rope_keys = 1
+    ws = torch.empty(max(16, tla.kivi_workspace_bytes(desc, longest)), dtype=torch.uint8, device="cuda")
+    out = torch.full_like(qd, float("nan"))
+    tla.kivi_paged_attention_decode_pre_rope(desc, out, qd, torch.from_numpy(pages_np).cuda(), ptd, kd, vd, btd, sld,
+                                             longest, dev(cos_t), dev(sin_t), tla.ROPE_ADJACENT, ws)
+    torch.cuda.synchronize()
+    want = orc.kivi_paged_attention(kc.q, orc.F16, pages_np, kc.page_tables, kc.k, kc.v, kc.tables, kc.lens,
+                                    kc.n_kv, kc.R, kc.scale, orc.GROUPED, bits, pre_rope=(cos_t, sin_t, tla.ROPE_ADJACENT))
+    assert_close(out, want, orc.F16, ATOL_KIVI, "uneven before RoPE")
+
+
 @pytest.mark.parametrize("H,n_kv", [(16, 8), (64, 8), (8, 8)])
 @pytest.mark.parametrize("gqa", [tla.GQA_GROUPED, tla.GQA_MODULO])
 def test_kivi_decode_group_sizes(H, n_kv, gqa):

@@ -852,8 +852,57 @@ int tl_kivi_append(const tl_kivi_desc* desc, const void* key, const void* value,
   return ok();
 }
 
-// rope: the _pre_rope entry points, whose workgroups take at most
-// tl::kivi_page_rot_cap(bits) pages
+// (sequence, kv head, 4-head slice) workgroups of one partition.
+static long kivi_items(const tl_kivi_desc* d) {
+  return (long)d->num_seqs * d->num_kv_heads * ((d->num_heads / d->num_kv_heads + 3) / 4);
+}
+
+// Pages of a partition that split `pages` evenly towards 512 workgroups.
+static int kivi_even_split(const tl_kivi_desc* d, int pages) {
+  const long items = kivi_items(d);
+  long want = items > 0 ? (512 + items - 1) / items : 1;
+  if (want < 1) want = 1;
+  if (want > pages) want = pages;
+  return (int)((pages + want - 1) / want);
+}
+
+// Pages that a workgroup takes at most: it stages their ids in LDS and, with
+// rope (the _pre_rope entry points), their rotations.
+static int kivi_page_cap(const tl_kivi_desc* d, bool rope) {
+  return rope ? std::min(tl::kKiviMaxWgPages, tl::kivi_page_rot_cap(kivi_bits(d))) : tl::kKiviMaxWgPages;
+}
+
+// The partitions of a batch: towards 512 workgroups, two per CU, as
+// kivi_even_split, except over short contexts, where a workgroup's start
+// (page ids, rotations) and the merge weigh more than what splitting evens
+// out between sequences of different lengths.
+//
+// us of the even split over us of this plan, the step of 32/8 heads, window
+// 128, on both sides of each line: equal lengths / the mean of five draws of
+// uneven ones (from a sixteenth of the longest); INT8 before RoPE, INT8, INT4
+// before RoPE, INT4.
+//   129 .. 511 items run single pass up to 48 pages, 24 for INT8 at 257 ..
+//   447.  18 sequences, 42 pages: 1.36/1.09, 1.19/1.00, 1.40/1.17, 1.33/1.15;
+//   33: 1.13/1.02, -, 1.24/1.05, 1.26/1.14; 36 of 20, INT8: 1.22/1.12.  Past
+//   it, 18 of 72: 1.15/0.89, 1.15/0.95, 1.18/0.97, 1.25/1.04; 36 of 42, INT8:
+//   1.05/0.97, 41 of 39 1.02/0.92.
+//   Up to 80 pages where the CUs have a workgroup each, or nearly (224 .. 256
+//   items), and at 4 bits up to 447 items: 28 of 72: 1.22/1.11, 1.24/1.14,
+//   1.24/1.17, 1.34/1.19; 32: 1.19/1.07, 1.16/1.22, 1.11/1.04, 1.22/1.18; 36,
+//   4 bits: 1.19/1.03, 1.14/1.09.  Past it, of 96: 28 1.17/1.00, 1.22/1.12,
+//   1.16/1.01, 1.27/1.09; 32 1.09/0.93, 1.13/1.11, 0.94/0.88, 1.15/1.01; 36, 8
+//   bits, of 72: 1.05/1.02, 0.99/0.94.
+//   Up to 100 pages with nearly two each (448 .. 511): 56 of 96: 1.15/1.15,
+//   1.05/0.99, 1.11/1.23, 1.17/1.21.
+//   64 .. 128 items: about one workgroup per CU, the last partition with
+//   fewer pages, by what its fp16 window and the append take beside pages (45
+//   at a window of 128, at most half the pages).  Up to 70 pages a partition
+//   with rope, 100 at 4 bits, 90 in two partitions at 8 bits and 24 in more.
+//   9 sequences of 86: 1.40/1.07, -, 1.40/1.07, 1.26/1.06; 14: 1.39/0.99,
+//   1.35/0.98, 1.46/1.03, 1.35/1.12; 16: 1.18/1.01, 1.18/1.04, 1.15/1.00,
+//   1.17/1.16; 10 of 42: 1.30/1.09, 1.13/1.00, 1.28/1.10, 1.16/1.05.  Past
+//   them, 16 of 124: 1.15/0.91 and 1.10/0.92 with rope; 14 of 246: 1.17/0.87
+//   and 1.27/0.82 without; 10 of 86, 8 bits in three: 1.06/0.90.
 static void kivi_plan(const tl_kivi_desc* d, int32_t max_ctx, bool rope, int* P, int* PP) {
   const int pages = tl::kivi_quantized_len(max_ctx, d->residual_length) / tl::kKiviPageTokens;
   int pp;
@@ -862,56 +911,39 @@ static void kivi_plan(const tl_kivi_desc* d, int32_t max_ctx, bool rope, int* P,
   } else if (d->partition_pages > 0) {
     pp = d->partition_pages;
   } else {
-    const int group = d->num_heads / d->num_kv_heads;
-    const long items = (long)d->num_seqs * d->num_kv_heads * ((group + 3) / 4);
-    long want = items > 0 ? (512 + items - 1) / items : 1;
-    if (want < 1) want = 1;
-    if (want > pages) want = pages;
-    pp = (int)((pages + want - 1) / want);
-    // Grids of an eighth of the CUs' workgroups and more do better with fewer
-    // partitions than 512 workgroups need: each costs its start (page ids,
-    // rotations) and the merge.  Below 144 items about one workgroup per CU,
-    // the last partition with fewer pages, by what its fp16 window and the
-    // append take beside pages (45 at a window of 128, at most half the
-    // pages); up to 256 items a single pass, as from 448 on and, at 4 bits, in
-    // between.  Longer contexts keep 512 workgroups, as INT4 at 256 items does
-    // with keys held before RoPE, where the rotation of a page, and not the
-    // start, is what counts.
-    // us, the step at 2900 tokens, INT8 before RoPE / INT8 / INT4 before RoPE
-    // / INT4 (32/8 heads, window 128): 16 sequences 46.1, 35.4, 40.4, 27.2
-    // before and 41.2, 30.7, 35.3, 23.4 now; 24: 64, 51, 56, 35 and 59, 41,
-    // 51, 29; 56: 107, 91, 81, 56 and 92, 86, 66, 48.  Past the lines: 32
-    // INT4 before RoPE 47.9 split, 51.2 single; 48 INT8 74 and 80; 20 of 8000
-    // tokens, INT8, 83 and 92.
+    pp = kivi_even_split(d, pages);
+    const long items = kivi_items(d);
     const bool int4 = kivi_bits(d) == 4;
-    if (items >= 64 && items < 144) {
+    if (items >= 64 && items <= 128) {
       const long parts = (256 + items / 2) / items;
       const long window = std::min<long>(10L * (d->residual_length + 16) / 32, pages / 2);
-      const long even = (pages + window + parts - 1) / parts;
-      if (even <= (int4 || rope ? 100 : 90)) pp = (int)std::min((long)pages, even);
-    } else if ((items >= 144 && items <= 256 && pages <= 192 && !(items == 256 && int4 && rope)) ||
-               (items >= 448 && items < 512 && pages <= 100) ||
-               (items > 256 && items < 448 && int4 && pages <= 100)) {
-      pp = pages;
+      const long part = std::min<long>(pages, (pages + window + parts - 1) / parts);
+      if (part <= (rope ? 70 : int4 ? 100 : parts == 2 ? 90 : 24)) pp = (int)part;
+    } else if (items > 128 && items < 512) {
+      const int single = items < 224 ? 48 : items <= 256 ? 80 : items < 448 ? (int4 ? 80 : rope ? 48 : 24) : 100;
+      if (pages <= single) pp = pages;
     }
   }
-  if (pp > tl::kKiviMaxWgPages) pp = tl::kKiviMaxWgPages;   // a workgroup stages its page ids in LDS
-  if (rope && pp > tl::kivi_page_rot_cap(kivi_bits(d))) pp = tl::kivi_page_rot_cap(kivi_bits(d));
+  pp = std::min(pp, kivi_page_cap(d, rope));
   *PP = pp;
   *P = pages > 0 ? (pages + pp - 1) / pp : 1;
 }
 
 size_t tl_kivi_workspace_bytes(const tl_kivi_desc* desc, int32_t max_context_len) {
   if (check_kivi(desc) != TL_OK || max_context_len < 0) return 0;
-  // the larger of the two plans, so that the size serves every entry point:
-  // either may run more partitions (the _pre_rope one past its pages per
-  // workgroup, the other where it alone keeps the split towards 512
-  // workgroups)
+  // the larger of the two plans, so that the size serves every entry point
   int P, P_rope, PP;
   kivi_plan(desc, max_context_len, false, &P, &PP);
   kivi_plan(desc, max_context_len, true, &P_rope, &PP);
   P = std::max(P, P_rope);
   if (P <= 1) return 0;
+  // and the even split's, which no plan exceeds: a size asked for a longer
+  // context holds where that split would do
+  if (desc->partition_pages == 0) {
+    const int pages = tl::kivi_quantized_len(max_context_len, desc->residual_length) / tl::kKiviPageTokens;
+    const int pp = std::min(kivi_even_split(desc, pages), kivi_page_cap(desc, true));
+    P = std::max(P, (pages + pp - 1) / pp);
+  }
   const size_t sh = (size_t)desc->num_seqs * desc->num_heads * P;
   return sh * desc->head_size * 4 + 2 * sh * 4;
 }
