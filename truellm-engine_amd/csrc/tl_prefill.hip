@@ -831,7 +831,7 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   static_assert(KV == Q || KV == Kind::FP8, "a 2-byte pool holds the q type");
   constexpr int BSE = BS >= kPfKeys ? kPfKeys : BS;       // keys of an iteration per block
   constexpr int BPI = kPfKeys / BSE;                      // pool blocks per iteration
-  constexpr int NKE = BS == 8 ? 2 : 1;                    // blocks of a 16-key run
+  constexpr int KR = BS == 8 ? 8 : 16;                    // keys of a staging run, which lies in one block
   constexpr int E = KV == Kind::FP8 ? 1 : 2;              // pool bytes per element
   using M = Mfma32<Q>;                                 // q.k
   using MP = Mfma32<Kind::F16>;                        // p.v (f16 for every type)
@@ -885,10 +885,16 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   };
 
   // Staging: a wavefront copies keys 32 wr .. + 31 of its group's iteration
-  // as units of 16 keys x 32 channels: lane l channel l % 32 of the unit and
-  // 8 keys, so that a load reads 1 KB (FP8: 512 B) contiguous in the pool at
-  // block sizes 16 and 32 (as prefill_kernel's).
-  constexpr int kRuns = kPfKeys / 16 / kSplitWaves, kUnits = 4;
+  // as units of KR keys x 512 / KR channels: lane l one channel of the unit
+  // and 8 keys, so that a load reads 1 KB (FP8: 512 B) contiguous in the pool
+  // at block sizes 8 (a whole block's keys, 64 channels), 16 and 32.  With
+  // prefill_kernel's units at block size 8 as well (16 keys in two blocks, a
+  // load for each whose other half is empty) the copies of 2-byte pools hold
+  // twice the registers and 224 to 244 bytes a lane go to scratch: bf16, 500
+  // queries of 1500 keys 58.2 us then, 32.6 so (prefill_kernel 66.6); 8
+  // prompts of 32 of 128 19.2, 11.8 (13.8).
+  constexpr int kUnitCh = 8 * kWave / KR, kRuns = kPfKeys / KR / kSplitWaves, kUnits = kPfHead / kUnitCh;
+  const int lane_ch = lane % kUnitCh, lane_tok = KR == 8 ? 0 : 8 * g;
   struct Fetched { u32x4 k[kRuns][kUnits], v[kRuns][kUnits]; int nv[kRuns]; };
   const int64_t head_bytes = (int64_t)kPfHead * BS * E;
   auto rsrc_of = [&](const char* pool, int pb) {
@@ -903,38 +909,19 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
       return u32x4{(uint32_t)w[0], (uint32_t)w[1], 0u, 0u};
     }
   };
-  auto run_key = [&](int r) { return 16 * (kRuns * wr + r); };
+  auto run_key = [&](int r) { return KR * (kRuns * wr + r); };
   // the copy's K (PART 0) or V (1)
   auto fetch = [&](int it, int entries, Fetched& f, auto part) {
     constexpr int PART = decltype(part)::value;
 #pragma unroll
     for (int r = 0; r < kRuns; ++r) {
-      int pb[NKE];
-#pragma unroll
-      for (int h = 0; h < NKE; ++h) pb[h] = block_at(it, entries, run_key(r) + 8 * h);
-      const int tok = run_key(r) + 8 * g;
-      if constexpr (PART == 1) {
-        const int pb_lane = NKE == 2 ? (g ? pb[NKE - 1] : pb[0]) : pb[0];
-        f.nv[r] = pb_lane >= 0 ? min(max(L - (it * kPfKeys + tok), 0), 8) : 0;
-      }
+      const int pb = block_at(it, entries, run_key(r)), tok = run_key(r) + lane_tok;
+      if constexpr (PART == 1) f.nv[r] = pb >= 0 ? min(max(L - (it * kPfKeys + tok), 0), 8) : 0;
       const int in_blk = BS > kPfKeys ? (int)((unsigned)(it * kPfKeys) % BS) + tok : tok % BS;
 #pragma unroll
-      for (int u = 0; u < kUnits; ++u) {
-        const char* pool = PART == 0 ? p.k_cache : p.v_cache;
-        const unsigned off = unsigned(E * ((32 * u + c32) * BS + in_blk));
-        u32x4 w;
-        if constexpr (NKE == 1) {
-          w = load_raw(rsrc_of(pool, pb[0]), off);
-        } else {
-          // each load serves one lane half; the other half's offset lies
-          // past the range (no memory request, zeros)
-          constexpr unsigned kPast = 0x40000000u;
-          const u32x4 a = load_raw(rsrc_of(pool, pb[0]), g == 0 ? off : kPast);
-          const u32x4 c = load_raw(rsrc_of(pool, pb[1]), g == 1 ? off : kPast);
-          w = u32x4{a.x | c.x, a.y | c.y, a.z | c.z, a.w | c.w};
-        }
-        (PART == 0 ? f.k : f.v)[r][u] = w;
-      }
+      for (int u = 0; u < kUnits; ++u)
+        (PART == 0 ? f.k : f.v)[r][u] = load_raw(rsrc_of(PART == 0 ? p.k_cache : p.v_cache, pb),
+                                                 unsigned(E * ((kUnitCh * u + lane_ch) * BS + in_blk)));
     }
   };
   const std::integral_constant<int, 0> kKeys;
@@ -942,18 +929,18 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   auto stage = [&](const Fetched& f) {
 #pragma unroll
     for (int r = 0; r < kRuns; ++r) {
-      const int tok = run_key(r) + 8 * g;
+      const int tok = run_key(r) + lane_tok;
 #pragma unroll
       for (int u = 0; u < kUnits; ++u)
-        *reinterpret_cast<u32x4*>(&sm.st.kt[grp][(32 * u + c32) * kKtStride + tok]) =
+        *reinterpret_cast<u32x4*>(&sm.st.kt[grp][(kUnitCh * u + lane_ch) * kKtStride + tok]) =
             KV == Kind::FP8 ? fp8x8_to<Q>(f.k[r][u]) : f.k[r][u];
     }
 #pragma unroll
     for (int r = 0; r < kRuns; ++r) {
-      const int tok = run_key(r) + 8 * g;
+      const int tok = run_key(r) + lane_tok;
 #pragma unroll
       for (int u = 0; u < kUnits; ++u) {
-        const int ch = 32 * u + c32;
+        const int ch = kUnitCh * u + lane_ch;
         // V slots at or past the sequence end may hold anything: zero them
         u4v v = __builtin_bit_cast(u4v, KV == Kind::FP8 ? fp8x8_to<Kind::F16>(f.v[r][u]) : f.v[r][u]);
         const int nv = f.nv[r];
