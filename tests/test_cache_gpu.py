@@ -248,3 +248,10 @@ def test_prompt_append_bit_exact(kind, code, n_kv, D, BS):
         assert np.array_equal(host_bits(q_out), q_ref)
     assert np.array_equal(host_bits(kcd), kc)
     assert np.array_equal(host_bits(vcd), vc)
+
+
+@pytest.mark.parametrize("kind", ["copy", "halves", "fp8"])
+@pytest.mark.parametrize("n_kv,D,BS", [(2, 64, 32), (8, 128, 32), (12, 128, 16), (12, 64, 64)])
+def test_prompt_append_tile_lengths(kind, n_kv, D, BS):
+    """Tiles of 8, 16 and 32 tokens, by the workgroups that the call makes; runs longer than a tile."""
+    test_prompt_append_bit_exact(kind, orc.BF16, n_kv, D, BS)

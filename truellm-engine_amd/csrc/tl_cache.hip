@@ -408,8 +408,8 @@ __global__ __launch_bounds__(64) void rope_rows_kernel(RopeCache a) {
 // Prompt-sized appends.  The element stores of reshape_copy_kernel and
 // rope_cache_kernel leave one 2-byte store per (token, channel), each
 // instruction over 64 lines of the pool.  Here a workgroup takes a tile of 32
-// consecutive tokens of one kv head, of K or of V, stages their rows in LDS
-// and writes the pool along the slots: where C = 16 / E tokens of the tile
+// (small calls: 16 or 8) consecutive tokens of one kv head, of K or of V,
+// stages their rows in LDS and writes the pool along the slots: where C = 16 / E tokens of the tile
 // fill an aligned 16-byte chunk, it is one store per channel, with the lanes
 // of a store over consecutive chunks of a block's rows; tokens that fill no
 // chunk are stored element by element, and no slot of another token is
@@ -425,8 +425,9 @@ __global__ __launch_bounds__(64) void rope_rows_kernel(RopeCache a) {
 // 16, rotated: 28.2 us (element stores: 93.7); 4096 tokens copied without
 // rotation 7.9 us (43.2), into FP8 pools 8.3 us (42.8).  Tokens that each lie
 // in a block of their own (a decode batch of more than 256 sequences) are
-// stored element by element as before: 512 of them copied 10.4 us (9.8),
-// 1024 17.1 (17.5).
+// stored element by element as before: 512 of them copied 10.2 us (10.2),
+// 1024 17.0 (17.8), in blocks of 32 slots 15.7 (14.8) and 28.2 (27.4); rotated
+// 11.8 (14.3), into FP8 pools 7.1 (13.5).
 struct TileAppend {
   const void* q; void* q_out;              // ROPE only
   const void* key; const void* value;
@@ -435,11 +436,13 @@ struct TileAppend {
   const float* cos_table; const float* sin_table;
   int num_tokens, num_heads, num_kv_heads, head_size, block_size, num_blocks, max_positions;
   int group;                               // slots of a segment's group
+  int tile;                                // tokens of a tile: 8, 16 or 32
   int kv_wgs;                              // workgroups over K and V; q's follow
   float k_mul, v_mul;                      // FP8 pools
 };
 
-constexpr int kTileTokens = 32, kTileThreads = 256, kTileRowPad = 8;
+constexpr int kTileTokens = 32;            // at most
+constexpr int kTileThreads = 256, kTileRowPad = 8;
 constexpr int kTileHeadsPerThread = 4;     // q heads of one token and rotation unit
 constexpr int kNoRope = -1;
 
@@ -542,7 +545,7 @@ __global__ __launch_bounds__(kTileThreads) void append_tiles_kernel(TileAppend a
     }
   }
   constexpr int E = KindInfo<POOL>::bytes, C = 16 / E;
-  const int h = (int)(blockIdx.x / 2) % a.num_kv_heads, t0 = (int)(blockIdx.x / 2) / a.num_kv_heads * kTileTokens;
+  const int h = (int)(blockIdx.x / 2) % a.num_kv_heads, t0 = (int)(blockIdx.x / 2) / a.num_kv_heads * a.tile;
   const bool is_v = blockIdx.x % 2;
   const int tid = threadIdx.x, lane = tid % kWave;
 
@@ -560,11 +563,11 @@ __global__ __launch_bounds__(kTileThreads) void append_tiles_kernel(TileAppend a
   const bool next = slot >= 0 && before >= 0 && before + 1 == slot && slot % a.group != 0;
   const uint64_t valid = __builtin_amdgcn_ballot_w64(slot >= 0);
   const uint64_t lead = valid & ~__builtin_amdgcn_ballot_w64(next);
-  constexpr uint64_t kIn = (1ull << kTileTokens) - 1;
-  if ((lead & kIn) == 0) return;
-  const int lo = __builtin_ctzll(lead & kIn);
+  const uint64_t in = (1ull << a.tile) - 1;
+  if ((lead & in) == 0) return;
+  const int lo = __builtin_ctzll(lead & in);
   // the tile's last segment ends before the first token past the tile that leads or is not written
-  const uint64_t stop = (lead | ~valid) & ~kIn;
+  const uint64_t stop = (lead | ~valid) & ~in;
   const int hi = stop ? __builtin_ctzll(stop) : kWave;
   const uint64_t mine = valid & (~0ull << lo) & (hi < kWave ? (1ull << hi) - 1 : ~0ull);
   // chunks: C tokens of one segment from an aligned slot on
@@ -726,8 +729,16 @@ template <Kind SRC, Kind POOL, int ROPE>
 int launch_tiles(TileAppend a, hipStream_t stream) {
   constexpr int E = KindInfo<POOL>::bytes;
   a.group = tile_group(a.block_size, E);
-  const int64_t tiles = ((int64_t)a.num_tokens + kTileTokens - 1) / kTileTokens;
-  const int64_t kv = tiles * a.num_kv_heads * 2;
+  // Shorter tiles where those of 32 tokens are fewer than the CUs: a tile of
+  // tokens that fill no chunk is a serial 4096 stores of an element.  2 heads,
+  // 257 tokens, each in a block of its own 5.6 us in tiles of 32, 4.1 of 8
+  // (reshape_copy_kernel 5.0), in runs of 4 5.2 and 3.7 (4.2), consecutive 3.6
+  // and 3.2 (4.1); 8 heads, 512 tokens, 10.6 in tiles of 32, 10.2 of 16 (10.2),
+  // consecutive 3.8 and 3.6 (9.4).  Past the line 8 heads, 900 consecutive,
+  // rotated 5.6 in tiles of 32, 7.0 of 16.
+  auto workgroups = [&](int tile) { return ((int64_t)a.num_tokens + tile - 1) / tile * a.num_kv_heads * 2; };
+  a.tile = workgroups(32) <= 64 ? 8 : workgroups(32) <= 256 ? 16 : kTileTokens;
+  const int64_t kv = workgroups(a.tile);
   int64_t grid = kv;
   if (ROPE != kNoRope) {
     const int64_t sets = (a.num_heads + kTileHeadsPerThread - 1) / kTileHeadsPerThread;
@@ -735,7 +746,7 @@ int launch_tiles(TileAppend a, hipStream_t stream) {
   }
   if (grid > 0x7fffffff) return 3;
   a.kv_wgs = (int)kv;
-  const size_t lds = (size_t)(kTileTokens + a.group - 1) * (a.head_size * E + kTileRowPad);
+  const size_t lds = (size_t)(a.tile + a.group - 1) * (a.head_size * E + kTileRowPad);
   hipLaunchKernelGGL((append_tiles_kernel<SRC, POOL, ROPE>), dim3((unsigned)grid), dim3(kTileThreads), lds, stream,
                      a);
   return hipGetLastError() == hipSuccess ? 0 : 5;
