@@ -537,7 +537,7 @@ __device__ __forceinline__ void rotate_q_tile(const TileAppend& a, int wg) {
 
 template <Kind SRC, Kind POOL, int ROPE>
 __global__ __launch_bounds__(kTileThreads) void append_tiles_kernel(TileAppend a) {
-  extern __shared__ char tile_rows[];
+  extern __shared__ __attribute__((aligned(16))) char tile_rows[];   // written 8 bytes at a time
   if constexpr (ROPE != kNoRope) {
     if ((int)blockIdx.x >= a.kv_wgs) {
       rotate_q_tile<SRC, ROPE>(a, blockIdx.x - a.kv_wgs);
