@@ -108,6 +108,28 @@ def test_vector_codec_equal_magnitudes(D, O, G):
     assert np.array_equal(host_bits(back).ravel(), orc.kivi_decompress(want, n, D, O, G).ravel())
 
 
+def test_vector_codec_more_vectors_than_one_launch():
+    """2^29 vectors and a few more of 2 channels (8 lanes each: 2^32 threads): the records and the values around
+    the launches' ends and at the end, against calls on those vectors alone."""
+    n, stride = (1 << 29) + 5, orc.kivi_compressed_bytes(2, 0, 2)
+    row = torch.randn(1 << 16, dtype=torch.float32, device="cuda").half()
+    x = row.repeat(2 * n // row.numel() + 1)[:2 * n]
+    x[-64:] = torch.arange(64, device="cuda").half()
+    rec = torch.zeros(n * stride, dtype=torch.uint8, device="cuda")
+    back = torch.zeros(2 * n, dtype=torch.float16, device="cuda")
+    print(f"case vec codec n={n}", flush=True)
+    tla.kivi_compress(x, rec, n, 2, 0, 2)
+    tla.kivi_decompress(rec, back, n, 2, 0, 2)
+    for a, b in ((0, 4096), ((1 << 28) - 2048, (1 << 28) + 2048), (n - 4096, n)):
+        some = torch.zeros((b - a) * stride, dtype=torch.uint8, device="cuda")
+        there = torch.zeros((b - a) * 2, dtype=torch.float16, device="cuda")
+        tla.kivi_compress(x[2 * a:2 * b].clone(), some, b - a, 2, 0, 2)
+        tla.kivi_decompress(some, there, b - a, 2, 0, 2)
+        torch.cuda.synchronize()
+        assert torch.equal(rec[a * stride:b * stride], some) and some.any()
+        assert torch.equal(back[2 * a:2 * b].view(torch.int16), there.view(torch.int16))
+
+
 def test_vector_codec_hand_derived_slot_order():
     """The kernel writes the outliers in the reference's selection-slot order
     (kivi_cache.cu:50-78), byte for byte against records derived by hand

@@ -665,25 +665,32 @@ __global__ __launch_bounds__(2 * kWave) void kivi_prefix_kernel(PageJob j) {
 
 int launch_kivi_vec(const void* in, void* out, int n_vecs, int head_dim, int n_outliers,
                     int group_size, int stride, bool compress, hipStream_t stream) {
-  const dim3 grid((unsigned)((n_vecs + kVecVecs - 1) / kVecVecs));
   const int rec_bytes = kivi_record_bytes(head_dim, n_outliers, group_size);
-  const void* kv = compress ? in : out;
-  const void* rec = compress ? out : in;
+  const uint16_t* kv = (const uint16_t*)(compress ? in : out);
+  const uint8_t* rec = (const uint8_t*)(compress ? out : in);
   const bool wide = head_dim % 8 == 0 && (uintptr_t)kv % 16 == 0;
   const bool dwords = stride % 4 == 0 && (uintptr_t)rec % 4 == 0;
-  if (compress) {
-    auto go = [&](auto spl) {
-      hipLaunchKernelGGL(kivi_vec_compress_kernel<decltype(spl)::value>, grid, dim3(kWave), 0, stream,
-                         (const uint16_t*)in, (uint8_t*)out, n_vecs, head_dim, n_outliers, group_size, stride,
-                         rec_bytes, wide, dwords);
-    };
-    if (n_outliers <= kVecLanes) go(std::integral_constant<int, 1>());
-    else if (n_outliers <= 2 * kVecLanes) go(std::integral_constant<int, 2>());
-    else if (n_outliers <= 4 * kVecLanes) go(std::integral_constant<int, 4>());
-    else go(std::integral_constant<int, 8>());
-  } else {
-    hipLaunchKernelGGL(kivi_vec_decompress_kernel, grid, dim3(kWave), 0, stream, (const uint8_t*)in, (uint16_t*)out,
-                       n_vecs, head_dim, n_outliers, group_size, stride, rec_bytes, wide, dwords);
+  // a launch of 2^32 threads or more (2^29 vectors) wraps
+  constexpr int kMost = 1 << 28;
+  for (int first = 0, n; first < n_vecs; first += n) {
+    n = min(n_vecs - first, kMost);
+    const dim3 grid((unsigned)((n + kVecVecs - 1) / kVecVecs));
+    const uint16_t* x = kv + (int64_t)first * head_dim;
+    const uint8_t* r = rec + (int64_t)first * stride;
+    if (compress) {
+      auto go = [&](auto spl) {
+        hipLaunchKernelGGL(kivi_vec_compress_kernel<decltype(spl)::value>, grid, dim3(kWave), 0, stream, x,
+                           const_cast<uint8_t*>(r), n, head_dim, n_outliers, group_size, stride, rec_bytes, wide,
+                           dwords);
+      };
+      if (n_outliers <= kVecLanes) go(std::integral_constant<int, 1>());
+      else if (n_outliers <= 2 * kVecLanes) go(std::integral_constant<int, 2>());
+      else if (n_outliers <= 4 * kVecLanes) go(std::integral_constant<int, 4>());
+      else go(std::integral_constant<int, 8>());
+    } else {
+      hipLaunchKernelGGL(kivi_vec_decompress_kernel, grid, dim3(kWave), 0, stream, r, const_cast<uint16_t*>(x), n,
+                         head_dim, n_outliers, group_size, stride, rec_bytes, wide, dwords);
+    }
   }
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
