@@ -255,3 +255,21 @@ def test_prompt_append_bit_exact(kind, code, n_kv, D, BS):
 def test_prompt_append_tile_lengths(kind, n_kv, D, BS):
     """Tiles of 8, 16 and 32 tokens, by the workgroups that the call makes; runs longer than a tile."""
     test_prompt_append_bit_exact(kind, orc.BF16, n_kv, D, BS)
+
+
+def test_prompt_append_more_tokens_than_tiles_can_launch():
+    """2^28 tokens of one head of 8 channels: in tiles that is 2^32 threads, more than a launch takes."""
+    T, D, BS = (1 << 28) + 24, 8, 8
+    N = T // BS
+    key = torch.arange(T * D // 8, dtype=torch.int32, device="cuda").view(torch.float16).repeat(5)[:T * D]
+    value = key.flip(0)
+    slots = torch.arange(T, dtype=torch.int32, device="cuda").view(N, BS).flip(0).reshape(-1).contiguous()
+    k = torch.zeros(N, 1, D, BS, dtype=torch.float16, device="cuda")
+    v = torch.zeros_like(k)
+    print(f"case prompt append T={T}", flush=True)
+    tla.reshape_and_cache_split(key.view(T, 1, D), value.view(T, 1, D), k, v, slots)
+    torch.cuda.synchronize()
+    for pool, src in ((k, key), (v, value)):
+        want = src.view(torch.int16).view(N, BS, D).flip(0)
+        for a in range(0, N, N // 7):
+            assert torch.equal(pool.view(torch.int16)[a:a + N // 7, 0].transpose(1, 2), want[a:a + N // 7])

@@ -714,13 +714,25 @@ int tile_group(int block_size, int elem) {
   return g * elem >= 16 ? g : 0;
 }
 
+// Workgroups over K and V in tiles of `tile` tokens, and over q.
+int64_t tile_kv_wgs(const TileAppend& a, int tile) {
+  return ((int64_t)a.num_tokens + tile - 1) / tile * a.num_kv_heads * 2;
+}
+int64_t tile_q_wgs(const TileAppend& a) {
+  const int64_t sets = (a.num_heads + kTileHeadsPerThread - 1) / kTileHeadsPerThread;
+  return (a.num_tokens * sets * (a.head_size / 16) + kTileThreads - 1) / kTileThreads;
+}
+
 // Whether append_tiles_kernel takes the call: whole 16-byte chunks in a
-// block, 16-byte aligned rows and tables, and rows that leave LDS for
-// several workgroups (63 rows of 512 bytes: 32 KiB).
+// block, 16-byte aligned rows and tables, rows that leave LDS for several
+// workgroups (63 rows of 512 bytes: 32 KiB), and fewer than 2^32 threads,
+// past which a launch wraps (rows below 128 channels take more of them here
+// than in the kernels that store elements).
 bool tile_shape(const TileAppend& a, int src_elem, int elem, bool rope) {
   auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   if (!al(a.key) || !al(a.value) || !al(a.k_cache) || !al(a.v_cache)) return false;
   if (rope && (!al(a.cos_table) || !al(a.sin_table) || !al(a.q) || !al(a.q_out))) return false;
+  if (tile_kv_wgs(a, kTileTokens) + (rope ? tile_q_wgs(a) : 0) >= (1ll << 32) / kTileThreads) return false;
   return a.block_size * elem % 16 == 0 && tile_group(a.block_size, elem) != 0 && a.head_size * elem <= 512 &&
          (int64_t)a.head_size * src_elem % 16 == 0 && a.head_size * elem % 8 == 0;
 }
@@ -736,19 +748,12 @@ int launch_tiles(TileAppend a, hipStream_t stream) {
   // and 3.2 (4.1); 8 heads, 512 tokens, 10.6 in tiles of 32, 10.2 of 16 (10.2),
   // consecutive 3.8 and 3.6 (9.4).  Past the line 8 heads, 900 consecutive,
   // rotated 5.6 in tiles of 32, 7.0 of 16.
-  auto workgroups = [&](int tile) { return ((int64_t)a.num_tokens + tile - 1) / tile * a.num_kv_heads * 2; };
-  a.tile = workgroups(32) <= 64 ? 8 : workgroups(32) <= 256 ? 16 : kTileTokens;
-  const int64_t kv = workgroups(a.tile);
-  int64_t grid = kv;
-  if (ROPE != kNoRope) {
-    const int64_t sets = (a.num_heads + kTileHeadsPerThread - 1) / kTileHeadsPerThread;
-    grid += (a.num_tokens * sets * (a.head_size / 16) + kTileThreads - 1) / kTileThreads;
-  }
-  if (grid > 0x7fffffff) return 3;
-  a.kv_wgs = (int)kv;
+  const int64_t full = tile_kv_wgs(a, kTileTokens);
+  a.tile = full <= 64 ? 8 : full <= 256 ? 16 : kTileTokens;
+  a.kv_wgs = (int)tile_kv_wgs(a, a.tile);
+  const unsigned grid = (unsigned)(a.kv_wgs + (ROPE != kNoRope ? tile_q_wgs(a) : 0));
   const size_t lds = (size_t)(a.tile + a.group - 1) * (a.head_size * E + kTileRowPad);
-  hipLaunchKernelGGL((append_tiles_kernel<SRC, POOL, ROPE>), dim3((unsigned)grid), dim3(kTileThreads), lds, stream,
-                     a);
+  hipLaunchKernelGGL((append_tiles_kernel<SRC, POOL, ROPE>), dim3(grid), dim3(kTileThreads), lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : 5;
 }
 
