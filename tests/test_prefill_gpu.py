@@ -352,3 +352,25 @@ def test_few_and_many_tiles_match_oracle(kv, BS, H, n_kv):
         tla.chunked_prefill(desc, out, q, cu, k, v, bt, sl, int(pc.q_lens.max()))
         torch.cuda.synchronize()
         assert_close(out, want, code, 1e-2 if kv == "fp8" else ATOL, f"prompts={prompts}")
+
+
+@pytest.mark.parametrize("BS", [8, 16, 64])
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+def test_prompts_within_one_iteration_of_keys(kv, BS):
+    """Prompts whose keys are all in the first 64, in tables no wider: one key group has them and writes the rows
+    without a merge.  Rows end inside a wavefront, on it and past the tile's first; keys on, before and past a
+    block's end."""
+    for shape in ([(16, 16)], [(2, 2), (33, 33)], [(64, 64), (5, 40), (1, 17)], [(31, 64), (1, 64), (17, 63)]):
+        if kv == "fp8":
+            pc, k8, v8, ks, vs = _fp8_case(inputs.SEEDS[1] + BS, shape, 16, 4, orc.BF16, BS)
+            print(f"case prefill one iteration fp8 BS={BS} {shape}", flush=True)
+            assert_close(_run_fp8(pc, k8, v8, ks, vs), _ref_fp8(pc), orc.BF16, 1e-2, f"{shape}")
+            continue
+        pc = PrefillCase(inputs.SEEDS[1] + BS, shape, 16, 4, orc.BF16, BS=BS, nan_unused=True)
+        q, k, v = dev(pc.q, orc.BF16), dev(pc.case.k_cache, orc.BF16), dev(pc.case.v_cache, orc.BF16)
+        out = torch.full_like(q, float("nan"))
+        desc = tla.make_prefill_desc(q, k, dev(pc.case.tables), pc.S, 4, pc.case.scale)
+        print(f"case prefill one iteration bf16 BS={BS} {shape}", flush=True)
+        tla.chunked_prefill(desc, out, q, dev(pc.cu), k, v, dev(pc.case.tables), dev(pc.lens), int(pc.q_lens.max()))
+        torch.cuda.synchronize()
+        assert_close(out, pc.ref(), orc.BF16, ATOL, f"{shape}")

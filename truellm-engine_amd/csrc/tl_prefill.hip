@@ -275,7 +275,7 @@ __global__ __launch_bounds__(NW * kWave) void prefill_kernel(PrefillParams pp) {
   const int L = p.seq_lens[seq];
   if (ql <= 0) return;
 
-  if (ql == 1) return;                                  // decode rows: prefill_decode_kernel
+  if (ql == 1) return;                                  // decode rows: decode_row
 
   // ---- prefill tile ----
   const int rows = ql * p.group;
@@ -867,7 +867,7 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
   int t_cur = table_read(grp), t_next = table_read(grp + kSplit);
   const int q0 = pp.cu_q_lens[seq], ql = pp.cu_q_lens[seq + 1] - q0;
   const int L = p.seq_lens[seq];
-  if (ql <= 1) return;                                 // decode rows: prefill_decode_kernel
+  if (ql <= 1) return;                                 // decode rows: decode_row
   const int rows = ql * p.group, row0 = tile * kSplitRows;
   if (row0 >= rows) return;
   const int wrow0 = row0 + wr * kPfRows, my_row = wrow0 + c32;
@@ -1101,15 +1101,52 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
     }
   };
 
-  // Every wavefront passes the same barriers, and every path leaves the same
-  // loads in flight: copies past the last iteration are empty (missing
-  // blocks, no traffic), and a group's iteration past it is all masked.  K's
-  // copy goes out before the scores are formed, V's after, when the
-  // registers of the K operands are free.
+  // sum of the row of lane c32 over the lane halves
+  auto row_sum = [&]() {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, l_part),
+                                                     __builtin_bit_cast(unsigned, l_part), false, false);
+    return __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
+  };
+  // factor of a row of the output (the sums carry 2^kPExp)
+  auto row_inverse = [&](float l) { return l > 0.f ? PvScale<KV>::kP * __builtin_amdgcn_rcpf(l) : 0.f; };
+  const float rg = 1.f / (float)p.group;               // rows of the output as in prefill_kernel
+  const int64_t obase = (int64_t)q0 * p.num_heads + (p.gqa_map ? kvh * p.group : kvh);
+  const int rmul = p.gqa_map ? 1 : p.num_kv_heads, qmul = p.gqa_map ? p.num_heads - p.group : 0;
+  const bool odd = (c32 & 1) != 0;
+  // rows 8 j + 4 g .. + 3, channel 32 c + c32, the row factors in s_row
+  auto put = [&](int j, int c, const float (&sum)[4]) {
+    const float4 i4 = *reinterpret_cast<const float4*>(&s_row[8 * j + 4 * g]);
+    const float inv[4] = {i4.x, i4.y, i4.z, i4.w};
+    float a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[i] = sum[i] * inv[i];
+      if constexpr (KV == Kind::FP8) a[i] *= p.v_scale;
+    }
+    // two channels per 4-byte store: lanes 2 k and 2 k + 1 swap one value
+#pragma unroll
+    for (int ip = 0; ip < 4; ip += 2) {
+      const int row = wrow0 + 8 * j + 4 * g + ip + (odd ? 1 : 0);
+      const int qr = (int)(((float)row + 0.5f) * rg);
+      const float got = dpp<kDppXor1>(odd ? a[ip] : a[ip + 1]);
+      if (row < rows)
+        *reinterpret_cast<uint32_t*>((uint16_t*)p.out + (obase + (int64_t)row * rmul + (int64_t)qr * qmul) * kPfHead +
+                                     32 * c + (c32 & ~1)) = odd ? M::pack(got, a[ip + 1]) : M::pack(a[ip], got);
+    }
+  };
+
+  // Every wavefront passes the same number of barriers: two in each round of
+  // kSplit iterations but the first, which has one.  A group without an
+  // iteration in the last round only passes them (a branch on that within the
+  // loop costs every wait for a copy: f16, 128 of 4000 keys 58.6 us, 55.7 so).
+  // Every path leaves the same loads in flight: copies past the last
+  // iteration are empty (missing blocks, no traffic).  K's copy goes out before
+  // the scores are formed, V's after, when the registers of the K operands are
+  // free.
   int it = grp;
 #pragma unroll 1
-  for (int base = 0; base < n_it; base += kSplit, it += kSplit) {
-    if (base > 0) __syncthreads();                     // the stage's last readers are done
+  for (; it < n_it; it += kSplit) {
+    if (it >= kSplit) __syncthreads();                 // the stage's last readers are done
     stage(f);
     const int t_mask = t_cur;
     t_cur = t_next;
@@ -1118,16 +1155,30 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
     __syncthreads();
     attend(it, t_mask, [&]() { fetch(it + kSplit, t_cur, f, kValues); });
   }
+  if (it - grp < n_it) {                               // group 0 ran this round
+    if (it >= kSplit) __syncthreads();
+    __syncthreads();
+  }
+
+  const float l = row_sum();
+  // One iteration (a prompt's first 64 keys): group 0 has the sums, nothing
+  // to merge.  bf16, 16 queries of 16 keys 8.1 us, 64 of 64 8.3 (through the
+  // merge 10.5 and 10.6, prefill_kernel 9.1 and 10.9).
+  if (n_it <= 1) {
+    if (grp != 0) return;
+    if (g == 0) s_row[c32] = row_inverse(l);
+    wave_sync();
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) put(j, c, {o[c][4 * j], o[c][4 * j + 1], o[c][4 * j + 2], o[c][4 * j + 3]});
+    return;
+  }
 
   // ---- merge: every group's rows on the common maximum ----
-  {
-    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, l_part),
-                                                     __builtin_bit_cast(unsigned, l_part), false, false);
-    const float l = __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
-    if (g == 0) {
-      sm.m[wave][c32] = m_used;
-      sm.l[wave][c32] = l;
-    }
+  if (g == 0) {
+    sm.m[wave][c32] = m_used;
+    sm.l[wave][c32] = l;
   }
   __syncthreads();                                     // the last stage's readers too
   float m_all = -INFINITY, l_all = 0.f;
@@ -1146,13 +1197,9 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
     for (int j = 0; j < 4; ++j)
       *reinterpret_cast<float4*>(sm.o[wave][c][j][lane]) =
           make_float4(o[c][4 * j], o[c][4 * j + 1], o[c][4 * j + 2], o[c][4 * j + 3]);
-  if (g == 0) s_row[c32] = l_all > 0.f ? PvScale<KV>::kP * __builtin_amdgcn_rcpf(l_all) : 0.f;   // the sums carry 2^kPExp
+  if (g == 0) s_row[c32] = row_inverse(l_all);
   __syncthreads();
 
-  const float rg = 1.f / (float)p.group;               // rows of the output as in prefill_kernel
-  const int64_t obase = (int64_t)q0 * p.num_heads + (p.gqa_map ? kvh * p.group : kvh);
-  const int rmul = p.gqa_map ? 1 : p.num_kv_heads, qmul = p.gqa_map ? p.num_heads - p.group : 0;
-  const bool odd = (c32 & 1) != 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     float a[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1161,27 +1208,12 @@ __global__ __launch_bounds__(kSplitNW * kWave) void prefill_split_kernel(Prefill
       const float4 w = *reinterpret_cast<const float4*>(sm.o[k * kSplitWaves + wr][grp][j][lane]);
       a[0] += w.x; a[1] += w.y; a[2] += w.z; a[3] += w.w;
     }
-    const float4 i4 = *reinterpret_cast<const float4*>(&s_row[8 * j + 4 * g]);
-    const float inv[4] = {i4.x, i4.y, i4.z, i4.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] *= inv[i];
-      if constexpr (KV == Kind::FP8) a[i] *= p.v_scale;
-    }
-    // two channels per 4-byte store: lanes 2 k and 2 k + 1 swap one value
-#pragma unroll
-    for (int ip = 0; ip < 4; ip += 2) {
-      const int row = wrow0 + 8 * j + 4 * g + ip + (odd ? 1 : 0);
-      const int qr = (int)(((float)row + 0.5f) * rg);
-      const float got = dpp<kDppXor1>(odd ? a[ip] : a[ip + 1]);
-      if (row < rows)
-        *reinterpret_cast<uint32_t*>((uint16_t*)p.out + (obase + (int64_t)row * rmul + (int64_t)qr * qmul) * kPfHead +
-                                     32 * grp + (c32 & ~1)) = odd ? M::pack(got, a[ip + 1]) : M::pack(a[ip], got);
-    }
+    put(j, grp, a);
   }
 }
 
-// The decode rows alone: calls without prefill tiles, or with few of them.
+// The decode rows alone: calls without prefill tiles, with many of them or with
+// many rows (rows_with_tiles).
 template <Kind Q, Kind KV, int BS, int NW>
 __global__ __launch_bounds__(NW * kWave) void prefill_decode_kernel(PrefillParams pp) {
   __shared__ __attribute__((aligned(16))) DecodeRowSmem<NW> sm;
@@ -1244,11 +1276,13 @@ int launch_prefill_bs(const PrefillParams& pp, int bs, unsigned grid, hipStream_
 }  // namespace
 
 // Calls of at most this many 256-row tiles take the split kernel: four times
-// the workgroups, then, still run in one round, one per CU.  Measured against
-// prefill_kernel (bf16, 32/8 heads, us): at 64 tiles, 500 of 1500 keys 29.1
-// against 55.0; past the line, at 128, 2 prompts of 512 of 1500 51.6 against
-// 56.6, 4 of 256 of 1024 41.9 against 40.5, 8 of 128 of 128 21.4 against
-// 14.4, and at 256 tiles 100 against 60.
+// the workgroups, then, still run in one round, one per CU.  us split and in
+// prefill_kernel, bf16, 32/8 heads, blocks of 16 (of 64) slots: at 64 tiles 500
+// of 1500 keys 29.0 and 55.0 (36.4 and 53.4), 8 prompts of 64 of 64 8.9 and
+// 11.5 (9.6 and 12.0); past the line, at 80, 600 of 1500 42.4 and 55.7 (54.2
+// and 54.3), 5 of 128 of 500 26.2 and 25.1 (32.6 and 25.2); at 128, 2 of 512 of
+// 1500 48.9 and 56.0 (62.7 and 54.8), 8 of 128 of 128 16.8 and 13.7 (18.5 and
+// 14.5); at 256, 8 of 256 of 256 36.6 and 20.2 (41.7 and 20.7).
 constexpr int kSplitMaxTiles = 64;
 
 int launch_prefill(const PrefillLaunch& a) {
@@ -1279,10 +1313,7 @@ int launch_prefill(const PrefillLaunch& a) {
   pp.dec_first = a.num_prefill_seqs > 0 ? a.num_prefill_seqs : 0;
   // prefill tiles exist only for q_len > 1
   pp.row_tiles = a.max_q_len > 1 ? (a.max_q_len * p.group + NW * kPfRows - 1) / (NW * kPfRows) : 0;
-  // (a table of at most 64 keys has one iteration and nothing to split: 16
-  // of 16 keys 9.4 us, 10.9 split)
-  pp.split = (int64_t)pp.row_tiles * pp.pf_seqs * a.num_kv_heads <= kSplitMaxTiles &&
-             (int64_t)a.max_blocks_per_seq * a.block_size > kPfKeys;
+  pp.split = (int64_t)pp.row_tiles * pp.pf_seqs * a.num_kv_heads <= kSplitMaxTiles;
   if (pp.split && pp.row_tiles) pp.row_tiles = (a.max_q_len * p.group + kSplitRows - 1) / kSplitRows;
   const unsigned grid = (unsigned)(pp.row_tiles * pp.pf_seqs * a.num_kv_heads);
   pp.pf_wgs = (int)grid;
