@@ -203,8 +203,8 @@ def _prompt_slots(rng, BS, spans):
 @pytest.mark.parametrize("n_kv,D,BS", [(2, 128, 16), (3, 64, 8), (1, 128, 24), (2, 112, 40), (1, 256, 64), (2, 128, 12)])
 def test_prompt_append_bit_exact(kind, code, n_kv, D, BS):
     """More than 256 tokens: whole 16-byte chunks of a block's rows where tokens fill them, elements elsewhere.
-    Prompts begin anywhere in a block and end a tile early, on it and past it; 12-slot blocks take the
-    general kernel."""
+    Prompts begin anywhere in a block and end a tile early, on it and past it; 12-slot blocks of 2-byte
+    elements take the general kernel."""
     if kind == "fp8" and code == orc.F32:
         pytest.skip("FP8 pools take 2-byte sources")
     rng = np.random.default_rng(D * BS + n_kv)
@@ -250,11 +250,14 @@ def test_prompt_append_bit_exact(kind, code, n_kv, D, BS):
     assert np.array_equal(host_bits(vcd), vc)
 
 
-@pytest.mark.parametrize("kind", ["copy", "halves", "fp8"])
-@pytest.mark.parametrize("n_kv,D,BS", [(2, 64, 32), (8, 128, 32), (12, 128, 16), (12, 64, 64)])
-def test_prompt_append_tile_lengths(kind, n_kv, D, BS):
-    """Tiles of 8, 16 and 32 tokens, by the workgroups that the call makes; runs longer than a tile."""
-    test_prompt_append_bit_exact(kind, orc.BF16, n_kv, D, BS)
+@pytest.mark.parametrize("kind", ["copy", "halves", "adjacent", "fp8"])
+@pytest.mark.parametrize("code", [orc.F16, orc.BF16, orc.F32])
+@pytest.mark.parametrize("n_kv,D,BS", [(2, 64, 32), (8, 128, 32), (12, 128, 16), (12, 64, 64), (20, 64, 8), (9, 112, 40),
+                                       (6, 256, 16)])
+def test_prompt_append_tile_lengths(kind, code, n_kv, D, BS):
+    """Tiles of 8, 16 and 32 tokens, by the workgroups that the call makes; runs longer than a tile; rotated calls
+    on both sides of their line."""
+    test_prompt_append_bit_exact(kind, code, n_kv, D, BS)
 
 
 def test_prompt_append_more_tokens_than_tiles_can_launch():

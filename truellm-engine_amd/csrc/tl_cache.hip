@@ -832,7 +832,13 @@ int launch_rope_cache(const RopeCache& a_in, hipStream_t stream) {
   // decode-sized calls: one wavefront per (token, kv head), whole block rows
   const bool rows = a.num_tokens <= kRowAppendMaxTokens && (a.block_size * E) % 16 == 0 && aligned &&
                     a.num_heads % a.num_kv_heads == 0;
-  if (a.num_tokens > kRowAppendMaxTokens) {
+  // Few rows (a shard's 1 or 2 kv heads) are waits for memory more than stores,
+  // of which rope_cache_kernel has fewer: 8/1 heads of 128, 257 tokens 4.5 us
+  // there, 5.2 in tiles, 600 4.9 and 5.3; 16/2, 300 4.8 and 5.3.  Past the line
+  // 16/2, 400 5.4 and 5.4, 600 7.1 and 5.5; 32/2, 257 5.9 and 5.5; 16/4, 257 5.7
+  // and 5.3.
+  const int64_t rotated = (int64_t)a.num_tokens * (a.num_heads + (int64_t)8 * a.num_kv_heads) * a.head_size;
+  if (a.num_tokens > kRowAppendMaxTokens && rotated >= 10000 * 128) {
     TileAppend ta = {};
     ta.q = a.q; ta.q_out = a.q_out; ta.key = a.key; ta.value = a.value;
     ta.k_cache = (char*)a.k_cache; ta.v_cache = (char*)a.v_cache;
