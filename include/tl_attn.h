@@ -608,7 +608,8 @@ int32_t tl_kivi_pass_runs(int32_t seq_len, int32_t n_kv_heads, int32_t head_dim,
  * pool with tl_reshape_and_cache); query i sits at position
  * seq_lens[s] - q_len + i and attends causally to keys 0 .. that position.
  * q_len == 1 rows are decode rows (after the tiles in one launch when they
- * are few, else a kernel of their own on the same stream).
+ * are few, else a kernel of their own on the same stream, with another order
+ * of its fp32 sums: the last bits of a row's output depend on the batch).
  * head_size 128, block_size any power of two 8..256 (CudaEngineConfig's
  * paged_kv_block_size, config_schema.h:68), dtype F16 or BF16 for q and out;
  * the pool holds dtype, or FP8 E4M3 codes with per-tensor scales

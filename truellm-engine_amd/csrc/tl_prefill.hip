@@ -40,7 +40,8 @@
 // v_scale (codes converted exactly to the q type for q.k and to f16 for
 // p.v as they are staged; k_scale folds into the score scale, v_scale into
 // the output).  Block sizes: any power of two 8 .. 256; a wavefront's 16-key
-// group lies in one block from 16 on, in two at 8 (one per lane half).
+// group lies in one block from 16 on, in two at 8 (one per lane half; the
+// split kernel copies block by block there).
 //
 // Nearest reference analogues: the per-token prefill of cuda_engine.cpp:842-860
 // and the dense attention of megakernel.cu:267-351; the reference has no
@@ -806,8 +807,8 @@ __global__ __launch_bounds__(NW * kWave) void prefill_kernel(PrefillParams pp) {
 // Bound by what a CU takes in: an iteration of its four groups is 128 KB from
 // L2 and through LDS for 64 rows (prefill_kernel: 32 KB for 256), so it pays
 // only while the other kernel leaves CUs idle.  f16, 32/8 heads, us, before
-// and after: 500 queries of 1500 keys 52.4 and 26.5; bf16: 256 of 256 17.0
-// and 11.0, 512 of 6000 187.6 and 88.6, 16 of 3000 95.7 and 47.7.
+// and after: 500 queries of 1500 keys 52.4 and 26.1; bf16: 256 of 256 17.2
+// and 11.1, 512 of 6000 188.3 and 94.9, 16 of 3000 96.3 and 46.0.
 constexpr int kSplit = 4;                    // key groups of a workgroup
 constexpr int kSplitWaves = 2;               // wavefronts (32 rows each) of a key group
 constexpr int kSplitRows = kSplitWaves * kPfRows;
